@@ -142,41 +142,19 @@ def _tet_scene(c, seed):
     mu, lam = sg.scenes.lame_from_young(E, NU)
     pairs, pair_x = np.zeros((0, 4), np.int32), None
     if c["pairs"]:
-        pairs, pair_x = _pairs(x, tris, c["pairs"], rng)
+        pairs, pair_x = sg.scenes.seed_pt_pairs_on(x, tris, c["pairs"], DHAT, [seed, 5])
     return dataclasses.replace(base, x=x, mu=mu, lam=lam, pairs=pairs, pair_x=pair_x,
                                rhs=rng.standard_normal(3 * base.n))
 
 
-def _cliques(tris, n, rng):
-    """A boundary vertex and a boundary triangle that does not hold it, n times."""
-    t = tris[rng.integers(0, len(tris), n)]
-    pv = tris[rng.integers(0, len(tris), n), 0]
-    touching = (t == pv[:, None]).any(1)
-    while touching.any():
-        t[touching] = tris[rng.integers(0, len(tris), int(touching.sum()))]
-        touching = (t == pv[:, None]).any(1)
-    return pv, t
-
-
-def _pairs(x, tris, n_pairs, rng):
-    """Seeded point-triangle pairs at d^2 ~ U(0, dhat^2) with their own local geometry."""
-    pv, t = _cliques(tris, n_pairs, rng)
-    bary = rng.uniform(0.1, 1.0, (n_pairs, 3))
-    bary /= bary.sum(1, keepdims=True)
-    a, b, d = x[t[:, 0]], x[t[:, 1]], x[t[:, 2]]
-    nrm = np.cross(b - a, d - a)
-    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
-    off = np.sqrt(np.maximum(rng.uniform(0, 1, n_pairs), 1e-6)) * DHAT * np.where(rng.uniform(size=n_pairs) < 0.5, -1, 1)
-    p = bary[:, :1] * a + bary[:, 1:2] * b + bary[:, 2:] * d + off[:, None] * nrm
-    return np.stack([-pv - 1, t[:, 0], t[:, 1], t[:, 2]], 1).astype(np.int32), np.stack([p, a, b, d], 1)
-
-
 def _contacts(c, tris, seed):
-    """(pairs, 4) vertices of seeded contact cliques over the boundary."""
+    """(pairs, 4) vertices of seeded contact cliques over the boundary: a vertex and a triangle that does not hold it."""
     if not c["pairs"]:
         return torch.zeros((0, 4), dtype=I64, device="cuda")
-    pv, t = _cliques(tris, c["pairs"], np.random.default_rng([seed, 2]))
-    return torch.from_numpy(np.concatenate([pv[:, None], t], 1).astype(np.int64)).cuda()
+    rest = _mesh(c["nx"], c["ny"], c["nz"])[0]
+    q = sg.scenes.seed_pt_pairs_on(rest, tris, c["pairs"], DHAT, [seed, 2])[0].astype(np.int64)
+    q[:, 0] = -q[:, 0] - 1
+    return torch.from_numpy(q).cuda()
 
 
 def _matrix(c, seed):
