@@ -1,28 +1,44 @@
-// Contact-pair generation (LBVH broad phase + distance-type narrow phase) and
+// Contact-pair generation (Morton-cluster broad phase + distance-type narrow phase) and
 // the barrier gradient/Hessian of every pair type.
 #pragma once
 #include "sgipc_internal.hpp"
 
 namespace sgipc {
 
-// Linear BVH over triangles (k = 3) or edges (k = 2): Morton-sorted leaves
-// (Karras 2012 radix tree), AABBs refitted bottom-up.  Node numbering: internal
-// nodes [0, n - 1), leaf of sorted position s at n - 1 + s; the root is node 0
-// (a single leaf when n == 1).
-struct Lbvh {
-    int n = 0;
-    DevBuf<double> box;       // 6 per node: lo xyz, hi xyz
-    DevBuf<double> leaf_box;  // 6 per primitive (primitive order)
-    DevBuf<double> scene;     // 6 + partial boxes of the reduction
-    DevBuf<uint64_t> keys, skeys;
-    DevBuf<int> idx, sidx;    // sidx[s] = primitive at sorted position s
-    DevBuf<int> child;        // 2 per internal node
-    DevBuf<int> parent;       // per node (-1 at the root)
-    DevBuf<int> flag;         // per internal node, refit arrivals
-    DevBuf<unsigned char> temp;
+// The three primitive sets of the broad phase: 0 faces, 1 edges, 2 points
+// (surface vertices).  Primitives are numbered set after set; in the sorted
+// order every set is padded to whole clusters of 64 slots and to whole tops
+// of 64 clusters.
+struct BroadSets {
+    int n[3] = {0, 0, 0};      // primitives
+    int slot0[3] = {0, 0, 0};  // first slot
+    int top0[3] = {0, 0, 0};   // first top
+    int slots = 0, tops = 0;
+    __host__ __device__ int start(int k) const { return k == 0 ? 0 : (k == 1 ? n[0] : n[0] + n[1]); }
+    __host__ __device__ int total() const { return n[0] + n[1] + n[2]; }
+    __host__ __device__ int set_of(int i) const { return i >= n[0] + n[1] ? 2 : (i >= n[0] ? 1 : 0); }
+    __host__ __device__ int set_of_slot(int q) const { return q >= slot0[2] ? 2 : (q >= slot0[1] ? 1 : 0); }
+    __host__ __device__ int slot_end(int k) const { return slot0[k] + (n[k] + 63) / 64 * 64; }
+    __host__ __device__ int n_tops(int k) const { return (n[k] + 4095) / 4096; }
+};
+
+// Morton-sorted primitives with float boxes of leaves, clusters and tops
+// (struct of arrays: lo xyz, hi xyz), each at least a float step outside the
+// FP64 boxes.
+struct BroadPhase {
+    BroadSets sets;
+    DevBuf<double> box;         // 6 per primitive: lo xyz, hi xyz
+    DevBuf<int> sidx;           // primitive (inside its set) at sorted position start(set) + p
+    DevBuf<float> leaf, l1, l2;
     // dir (optional): boxes swept to x - alpha dir
-    void build(hipStream_t s, const double* x, const uint32_t* prims, int n_prims, int k, const double* dir = nullptr,
-               double alpha = 0.0);
+    void build(hipStream_t s, const double* x, const uint32_t* faces, int n_faces, const uint32_t* edges, int n_edges,
+               const uint32_t* points, int n_points, const double* dir, double alpha);
+
+  private:
+    DevBuf<double> part_;
+    DevBuf<uint32_t> keys_, skeys_;
+    DevBuf<int> idx_;
+    DevBuf<unsigned char> temp_;
 };
 
 // Counts of the reference's _cpNum: [0] pairs, [1] unused, [2] point-point,
@@ -61,13 +77,13 @@ class ContactDetector {
     int last_total = 0;
 
   private:
-    Lbvh fbvh_, ebvh_;
-    DevBuf<int> cnt_, off_, err_;
+    BroadPhase broad_;
+    long raw_cap_ = 0;  // entries of the unsorted pair buffer
+    DevBuf<int> cnt_, total_;
     DevBuf<uint64_t> rkey_, rkey_sorted_;
     DevBuf<int> rid_, rid_sorted_;
     DevBuf<int4> rpair_;
-    DevBuf<int> rcls_;
-    DevBuf<int> flags_, scan_;
+    DevBuf<uint64_t> cls_, cls_scan_;
     DevBuf<unsigned char> temp_;
     DevBuf<double> vals_;
     StepReducer red_;
