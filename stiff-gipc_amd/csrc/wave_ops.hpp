@@ -8,6 +8,14 @@ namespace sgipc {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// orders a wave's LDS writes before its lanes' later reads
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
 {
