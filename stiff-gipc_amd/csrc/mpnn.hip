@@ -125,44 +125,66 @@ __global__ void k_g_blocks(const uint64_t* __restrict__ sk, const int* __restric
 }
 
 // ------------------------------------------------------------------ layers
-// Y = Ahat V on 64 channels: one wave per node (lanes = channels), so a
-// launch keeps thousands of independent neighbour walks in flight.
+// Workgroup b of the n workgroups of a gather -> its place in the order
+// (sample, node): the 8 XCDs take workgroups in turn, so XCD b % 8 gets one
+// contiguous run, i.e. whole samples or stretches of neighbouring nodes whose
+// rows its own L2 then holds (a sample's 64 channels are 6 MB at 8k nodes).
+__device__ __forceinline__ int xcd_run(int b, int n)
+{
+    const int x = b & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (b >> 3);
+}
+
+// sum over node i's row of Ahat_ij (3 x 64 rows of src at row stride ld):
+// 16 lanes take 4 channels each, the wave's 4 groups every fourth neighbour
+// (4 load chains in flight); the groups are added in a fixed order and every
+// lane returns channels 4 (lane & 15) .. + 3.  One channel per lane and one
+// chain per wave, workgroups dealt over the XCDs: k_spmm64 235 and
+// k_bwd_gather 278 us on 16 samples of 8k nodes; this 170 and 191 us.
+__device__ __forceinline__ void gather64(const int* __restrict__ rp, const int* __restrict__ colx,
+                                         const float* __restrict__ blk, int i, const float* __restrict__ src, int ld,
+                                         f32x4 a[3])
+{
+    const int lane = threadIdx.x & 63, c4 = 4 * (lane & 15);
+    a[0] = a[1] = a[2] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int e1 = rp[i + 1];
+#pragma unroll 2
+    for (int e = rp[i] + (lane >> 4); e < e1; e += 4) {
+        const float* b = blk + 9L * e;
+        const float* v = src + 3L * colx[e] * ld + c4;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(v);
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(v + ld);
+        const f32x4 x2 = *reinterpret_cast<const f32x4*>(v + 2 * ld);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[0][k] += b[0] * x0[k] + b[1] * x1[k] + b[2] * x2[k];
+            a[1][k] += b[3] * x0[k] + b[4] * x1[k] + b[5] * x2[k];
+            a[2][k] += b[6] * x0[k] + b[7] * x1[k] + b[8] * x2[k];
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[d][k] += __shfl_xor(a[d][k], 16, 64);
+            a[d][k] += __shfl_xor(a[d][k], 32, 64);
+        }
+}
+
+// Y = Ahat V on 64 channels: one wave per node of every sample.
 __global__ __launch_bounds__(256) void k_spmm64(int n, const int* __restrict__ rp, const int* __restrict__ colx,
                                                 const float* __restrict__ blk, const float* __restrict__ V,
                                                 float* __restrict__ Y)
 {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int ch = threadIdx.x & 63;
+    const int w = xcd_run(blockIdx.x, gridDim.x), nb = (n + 3) / 4;
+    const int i = (w % nb) * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, d = lane >> 4;
     if (i >= n) return;
-    const long sbase = (long)blockIdx.y * 3 * n;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-    const int e1 = rp[i + 1];
-    int e = rp[i];
-    for (; e + 1 < e1; e += 2) {  // two neighbours per step: two load chains in flight
-        const int j0 = colx[e], j1 = colx[e + 1];
-        const float* b0 = blk + 9L * e;
-        const float* b1 = b0 + 9;
-        const float* v0 = V + (sbase + 3L * j0) * C + ch;
-        const float* v1 = V + (sbase + 3L * j1) * C + ch;
-        const float x0 = v0[0], x1 = v0[C], x2 = v0[2 * C];
-        const float y0 = v1[0], y1 = v1[C], y2 = v1[2 * C];
-        a0 += b0[0] * x0 + b0[1] * x1 + b0[2] * x2 + b1[0] * y0 + b1[1] * y1 + b1[2] * y2;
-        a1 += b0[3] * x0 + b0[4] * x1 + b0[5] * x2 + b1[3] * y0 + b1[4] * y1 + b1[5] * y2;
-        a2 += b0[6] * x0 + b0[7] * x1 + b0[8] * x2 + b1[6] * y0 + b1[7] * y1 + b1[8] * y2;
-    }
-    if (e < e1) {
-        const int j = colx[e];
-        const float* b = blk + 9L * e;
-        const float* vj = V + (sbase + 3L * j) * C + ch;
-        const float x0 = vj[0], x1 = vj[C], x2 = vj[2 * C];
-        a0 += b[0] * x0 + b[1] * x1 + b[2] * x2;
-        a1 += b[3] * x0 + b[4] * x1 + b[5] * x2;
-        a2 += b[6] * x0 + b[7] * x1 + b[8] * x2;
-    }
-    float* y = Y + (sbase + 3L * i) * C + ch;
-    y[0] = a0;
-    y[C] = a1;
-    y[2 * C] = a2;
+    const long sbase = (long)(w / nb) * 3 * n;
+    f32x4 a[3];
+    gather64(rp, colx, blk, i, V + sbase * C, C, a);
+    if (d < 3)
+        *reinterpret_cast<f32x4*>(Y + (sbase + 3L * i + d) * C + 4 * (lane & 15)) = d == 0 ? a[0] : (d == 1 ? a[1] : a[2]);
 }
 
 // Y = Ahat X on the 3 input features: one wave per node, lanes over the
@@ -391,21 +413,27 @@ __global__ __launch_bounds__(256) void k_bwd_dydu(int n, const float* __restrict
         const int rr = q >> 3, cc = (q & 7) * 8;
         *reinterpret_cast<u32x4*>(&sW[rr * kDld + cc]) = *reinterpret_cast<const u32x4*>(&Wn[rr * C + cc]);
     }
-    for (int q = t; q < kRows * C; q += 256) {
-        const int row = q / C, c = q % C;
-        uint16_t h = 0;
+#pragma unroll
+    for (int q = t; q < kRows * C / 4; q += 256) {
+        const int row = q / (C / 4), c = 4 * (q % (C / 4));
+        uint2 h = make_uint2(0u, 0u);
         if (row < rows_valid) {
             const long g = (sbase + 3L * node0 + row) * C + c;
-            const float d = (linear || Y[g] > 0.f) ? G[g] : 0.f;
-            h = f2bf(d);
-            dYout[g] = h;
+            const f32x4 gv = *reinterpret_cast<const f32x4*>(G + g), yv = *reinterpret_cast<const f32x4*>(Y + g);
+            uint16_t b[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) b[k] = f2bf((linear || yv[k] > 0.f) ? gv[k] : 0.f);
+            h = make_uint2(b[0] | ((uint32_t)b[1] << 16), b[2] | ((uint32_t)b[3] << 16));
+            *reinterpret_cast<uint2*>(dYout + g) = h;
         }
-        sD[row * kDld + c] = h;
+        *reinterpret_cast<uint2*>(&sD[row * kDld + c]) = h;
     }
     __syncthreads();
     const int lr = lane & 15;
     const int lk = (lane >> 4) * 8;
-    // 6 row tiles x 8 column tiles; wave wv takes column tiles 2wv, 2wv+1
+    // 6 row tiles x 8 column tiles; wave wv takes column tiles 2wv, 2wv+1.  W
+    // is the left operand, so a lane holds 4 consecutive columns of one row
+    // (16-byte stores, and 16-byte loads above: 168 -> 84 us on 383k rows)
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) {
         const int n0 = 16 * (2 * wv + ct);
@@ -414,49 +442,43 @@ __global__ __launch_bounds__(256) void k_bwd_dydu(int n, const float* __restrict
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kk = 0; kk < C / 32; ++kk) {
-                const bf16x8 av = ld8(&sD[(16 * mt + lr) * kDld + 32 * kk + lk]);
-                const bf16x8 bv = ld8(&sW[(n0 + lr) * kDld + 32 * kk + lk]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+                const bf16x8 dv = ld8(&sD[(16 * mt + lr) * kDld + 32 * kk + lk]);
+                const bf16x8 wvv = ld8(&sW[(n0 + lr) * kDld + 32 * kk + lk]);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wvv, dv, acc, 0, 0, 0);
             }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int row = 16 * mt + (lane >> 4) * 4 + j;
-                if (row < rows_valid) dU[(sbase + 3L * node0 + row) * 2 * C + n0 + lr] = acc[j];
-            }
+            const int row = 16 * mt + lr;
+            if (row < rows_valid)
+                *reinterpret_cast<f32x4*>(dU + (sbase + 3L * node0 + row) * 2 * C + n0 + (lane >> 4) * 4) = acc;
         }
     }
 }
 
-// G_new = G + dU[:, :C] + Ahat dU[:, C:] (one wave per node, lanes = channels).
+// G_new = G + dU[:, :C] + Ahat dU[:, C:] (one wave per node of every sample).
 __global__ __launch_bounds__(256) void k_bwd_gather(int n, const int* __restrict__ rp, const int* __restrict__ colx,
                                                     const float* __restrict__ blk, const float* __restrict__ G,
                                                     const float* __restrict__ dU, float* __restrict__ Gn)
 {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int ch = threadIdx.x & 63;
+    const int w = xcd_run(blockIdx.x, gridDim.x), nb = (n + 3) / 4;
+    const int i = (w % nb) * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, d = lane >> 4, c4 = 4 * (lane & 15);
     if (i >= n) return;
-    const long sbase = (long)blockIdx.y * 3 * n;
-    float a[3] = {0.f, 0.f, 0.f};
-    for (int e = rp[i]; e < rp[i + 1]; ++e) {
-        const int j = colx[e];
-        const float* b = blk + 9L * e;
-        const float* uj = dU + (sbase + 3L * j) * 2 * C + C + ch;
-        const float x0 = uj[0], x1 = uj[2 * C], x2 = uj[4 * C];
-        a[0] += b[0] * x0 + b[1] * x1 + b[2] * x2;
-        a[1] += b[3] * x0 + b[4] * x1 + b[5] * x2;
-        a[2] += b[6] * x0 + b[7] * x1 + b[8] * x2;
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
+    const long sbase = (long)(w / nb) * 3 * n;
+    f32x4 a[3];
+    gather64(rp, colx, blk, i, dU + sbase * 2 * C + C, 2 * C, a);
+    if (d < 3) {
         const long row = sbase + 3L * i + d;
-        Gn[row * C + ch] = G[row * C + ch] + dU[row * 2 * C + ch] + a[d];
+        const f32x4 g = *reinterpret_cast<const f32x4*>(G + row * C + c4);
+        const f32x4 u = *reinterpret_cast<const f32x4*>(dU + row * 2 * C + c4);
+        *reinterpret_cast<f32x4*>(Gn + row * C + c4) = g + u + (d == 0 ? a[0] : (d == 1 ? a[1] : a[2]));
     }
 }
 
 // First layer: dW_in[g][c] partial = sum_rows X[row][g] (G + dU_self)[row][c]
 //                                    + (Ahat X)[row][g] dU_nb[row][c]
-__global__ __launch_bounds__(256) void k_bwd_win(int n, const int* __restrict__ rp, const int* __restrict__ colx,
-                                                 const float* __restrict__ blk, const float* __restrict__ X,
+// over 256-row chunks; Ahat X as the forward pass left it (forming it again
+// from the graph for every channel took 347 us on 16 samples of 8k nodes,
+// reading it 78 us).
+__global__ __launch_bounds__(256) void k_bwd_win(long rows, const float* __restrict__ X, const float* __restrict__ AX,
                                                  const float* __restrict__ G, const float* __restrict__ dU,
                                                  float* __restrict__ part)
 {
@@ -464,41 +486,24 @@ __global__ __launch_bounds__(256) void k_bwd_win(int n, const int* __restrict__ 
     const int t = threadIdx.x;
     const int ch = t & 63;
     const int wv = t >> 6;
-    const int node0 = blockIdx.x * kMpnnTile;
-    const long sbase = (long)blockIdx.y * 3 * n;
+    const long r0 = (long)blockIdx.x * 256;
     float acc[3] = {0.f, 0.f, 0.f};
-    for (int m = 0; m < kMpnnTile / 4; ++m) {
-        const int i = node0 + wv + 4 * m;
-        if (i >= n) break;
-        float ax[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int e = rp[i]; e < rp[i + 1]; ++e) {
-            const int j = colx[e];
-            const float* b = blk + 9L * e;
-            const float* xj = X + (sbase + 3L * j) * 3;
+#pragma unroll 8
+    for (int k = wv; k < 256; k += 4) {
+        const long row = r0 + k;
+        if (row >= rows) break;
+        const float gs = G[row * C + ch] + dU[row * 2 * C + ch];
+        const float gn = dU[row * 2 * C + C + ch];
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int f = 0; f < 3; ++f)
-#pragma unroll
-                    for (int g = 0; g < 3; ++g) ax[3 * d + g] += b[3 * d + f] * xj[3 * f + g];
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const long row = sbase + 3L * i + d;
-            const float gs = G[row * C + ch] + dU[row * 2 * C + ch];
-            const float gn = dU[row * 2 * C + C + ch];
-#pragma unroll
-            for (int g = 0; g < 3; ++g) acc[g] += X[row * 3 + g] * gs + ax[3 * d + g] * gn;
-        }
+        for (int g = 0; g < 3; ++g) acc[g] += X[row * 3 + g] * gs + AX[row * 3 + g] * gn;
     }
 #pragma unroll
     for (int g = 0; g < 3; ++g) sm[(wv * 3 + g) * C + ch] = acc[g];
     __syncthreads();
     if (t < 3 * C) {
         const int g = t / C, c = t % C;
-        const long b = (long)blockIdx.y * gridDim.x + blockIdx.x;
-        part[b * 3 * C + t] = ((sm[(0 * 3 + g) * C + c] + sm[(1 * 3 + g) * C + c]) + sm[(2 * 3 + g) * C + c]) +
-                              sm[(3 * 3 + g) * C + c];
+        part[(long)blockIdx.x * 3 * C + t] =
+            ((sm[(0 * 3 + g) * C + c] + sm[(1 * 3 + g) * C + c]) + sm[(2 * 3 + g) * C + c]) + sm[(3 * 3 + g) * C + c];
     }
 }
 
@@ -519,19 +524,38 @@ __global__ __launch_bounds__(256) void k_dw(long rows, const uint16_t* __restric
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // a thread moves 4 rows x 4 columns at a time: four 8-byte loads, turned in
+    // registers, four 8-byte LDS writes; the next chunk's loads are in flight
+    // while this one is multiplied (383k rows: 145 -> 49 us against 2-byte
+    // transposed writes)
+    const int ur = 4 * (t >> 5), uc = 4 * (t & 31);  // of the 32 x 128 chunk of U
+    const int dr = 4 * (t >> 4), dc = 4 * (t & 15);  // of the 32 x 64 chunk of dY (threads < 128)
+    uint2 un[4], dn[4];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const long gu = r0 + k0 + ur + r, gd = r0 + k0 + dr + r;
+            un[r] = gu < rows ? *reinterpret_cast<const uint2*>(U + gu * 2 * C + uc) : make_uint2(0u, 0u);
+            if (t < 128) dn[r] = gd < rows ? *reinterpret_cast<const uint2*>(dY + gd * C + dc) : make_uint2(0u, 0u);
+        }
+    };
+    auto turn = [](const uint2 v[4], uint16_t* __restrict__ dst) {  // dst[col * 40 + row]
+        *reinterpret_cast<uint2*>(dst) =
+            make_uint2((v[0].x & 0xFFFFu) | (v[1].x << 16), (v[2].x & 0xFFFFu) | (v[3].x << 16));
+        *reinterpret_cast<uint2*>(dst + 40) =
+            make_uint2((v[0].x >> 16) | (v[1].x & 0xFFFF0000u), (v[2].x >> 16) | (v[3].x & 0xFFFF0000u));
+        *reinterpret_cast<uint2*>(dst + 80) =
+            make_uint2((v[0].y & 0xFFFFu) | (v[1].y << 16), (v[2].y & 0xFFFFu) | (v[3].y << 16));
+        *reinterpret_cast<uint2*>(dst + 120) =
+            make_uint2((v[0].y >> 16) | (v[1].y & 0xFFFF0000u), (v[2].y >> 16) | (v[3].y & 0xFFFF0000u));
+    };
+    fetch(0);
     for (int k0 = 0; k0 < kDwRows; k0 += 32) {
         __syncthreads();
-        for (int q = t; q < 32 * 2 * C; q += 256) {
-            const int row = q / (2 * C), u = q % (2 * C);
-            const long g = r0 + k0 + row;
-            sUT[u * 40 + row] = g < rows ? U[g * 2 * C + u] : (uint16_t)0;
-        }
-        for (int q = t; q < 32 * C; q += 256) {
-            const int row = q / C, c = q % C;
-            const long g = r0 + k0 + row;
-            sDT[c * 40 + row] = g < rows ? dY[g * C + c] : (uint16_t)0;
-        }
+        turn(un, sUT + uc * 40 + ur);
+        if (t < 128) turn(dn, sDT + dc * 40 + dr);
         __syncthreads();
+        if (k0 + 32 < kDwRows) fetch(k0 + 32);
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
             const int m0 = 16 * (2 * wv + a);
@@ -555,13 +579,23 @@ __global__ __launch_bounds__(256) void k_dw(long rows, const uint16_t* __restric
             }
 }
 
-// out[p] (+)= sum_b part[b][p], b in fixed order.
-__global__ void k_reduce_parts(const float* __restrict__ part, int nb, int np, float* __restrict__ out)
+// out[p] = sum_b part[b][p] in a fixed order (np a multiple of 64): a
+// workgroup takes 64 outputs, its 16 waves every 16th partial, in FP64.  One
+// thread per output left at most 32 workgroups to walk ~1000 partials one
+// load at a time: 232 to 1021 us per call against 8.
+__global__ __launch_bounds__(1024) void k_reduce_parts(const float* __restrict__ part, int nb, int np,
+                                                       float* __restrict__ out)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
+    __shared__ double sm[16][64];
+    const int p = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += (double)part[(long)b * np + p];
+#pragma unroll 8
+    for (int b = w; b < nb; b += 16) s += (double)part[(long)b * np + p];
+    sm[w][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (w != 0) return;
+#pragma unroll
+    for (int k = 1; k < 16; ++k) s += sm[k][threadIdx.x];
     out[p] = (float)s;
 }
 
@@ -738,6 +772,7 @@ void Mpnn::forward(hipStream_t st, const CoarseGraph& g, const float* X, int S, 
     AV_.reserve((size_t)rows * C);
     const dim3 grid((g.n + kMpnnTile - 1) / kMpnnTile, S);
     const dim3 gw((g.n + 3) / 4, S);  // one wave per node
+    const int gs = (int)gw.x * S;
     const float* w_in = w_.get();
     const float* w_out = w_.get() + 3 * C + (long)L * 2 * C * C;
     const float* vin = nullptr;
@@ -746,7 +781,7 @@ void Mpnn::forward(hipStream_t st, const CoarseGraph& g, const float* X, int S, 
         float* vout = V_[(l + 1) & 1].get();
         const bool first = l == 0, last = l == L - 1;
         if (first) k_spmm3<<<gw, 256, 0, st>>>(g.n, g.row_ptr.get(), g.col.get(), g.blk.get(), X, AV_.get(), done);
-        else k_spmm64<<<gw, 256, 0, st>>>(g.n, g.row_ptr.get(), g.col.get(), g.blk.get(), vin, AV_.get());
+        else k_spmm64<<<gs, 256, 0, st>>>(g.n, g.row_ptr.get(), g.col.get(), g.blk.get(), vin, AV_.get());
         SGIPC_LAUNCH_CHECK();
 #define SGIPC_LAYER(F, LA)                                                                                     \
     k_layer<F, LA, false><<<grid, 256, 0, st>>>(g.n, AV_.get(), vin, X, w_in, wt, LA ? nullptr : vout, w_out, chat, \
@@ -771,18 +806,20 @@ double Mpnn::loss_grad(hipStream_t st, const CoarseGraph& g, const float* X, con
     reserve_train(rows, tiles * S);
     const dim3 grid(tiles, S);
     const dim3 gw((n + 3) / 4, S);  // one wave per node
+    const int gs = (int)gw.x * S;
     const float* w_in = w_.get();
     const float* w_out = w_.get() + 3 * C + (long)L * 2 * C * C;
     AV_.reserve((size_t)rows * C);
-    // forward, keeping U, Y and every V
+    AX_.reserve((size_t)rows * 3);
+    // forward, keeping U, Y, every V and Ahat X
     for (int l = 0; l < L; ++l) {
         const uint16_t* wt = wt_.get() + (long)l * 2 * C * C;
         const bool first = l == 0, last = l == L - 1;
-        if (first) k_spmm3<<<gw, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), X, AV_.get(), nullptr);
-        else k_spmm64<<<gw, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), V_[l].get(), AV_.get());
+        if (first) k_spmm3<<<gw, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), X, AX_.get(), nullptr);
+        else k_spmm64<<<gs, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), V_[l].get(), AV_.get());
         SGIPC_LAUNCH_CHECK();
 #define SGIPC_LAYER(F, LA)                                                                                   \
-    k_layer<F, LA, true><<<grid, 256, 0, st>>>(n, AV_.get(), V_[l].get(), X, w_in, wt, V_[l + 1].get(), w_out, \
+    k_layer<F, LA, true><<<grid, 256, 0, st>>>(n, F ? AX_.get() : AV_.get(), V_[l].get(), X, w_in, wt, V_[l + 1].get(), w_out, \
                                                chat_.get(), g.s.get(), nullptr, U_[l].get(), Y_[l].get(),   \
                                                linear_, nullptr)
         if (first && last) SGIPC_LAYER(true, true);
@@ -797,7 +834,7 @@ double Mpnn::loss_grad(hipStream_t st, const CoarseGraph& g, const float* X, con
     const int gl = g256(nodes);
     const int n_dec = g256(rows);
     const int n_dw = (int)((rows + kDwRows - 1) / kDwRows);
-    const int n_win = tiles * S;
+    const int n_win = g256(rows);
     const long part_need = std::max({(long)gl, (long)n_dec * C, (long)n_dw * 2 * C * C, (long)n_win * 3 * C});
     part_.reserve(part_need);
     DevBuf<double>& lp = lpart_;
@@ -812,7 +849,7 @@ double Mpnn::loss_grad(hipStream_t st, const CoarseGraph& g, const float* X, con
     SGIPC_LAUNCH_CHECK();
     float* g_win = grad;
     float* g_wout = grad + 3 * C + (long)L * 2 * C * C;
-    k_reduce_parts<<<1, C, 0, st>>>(part_.get(), n_dec, C, g_wout);
+    k_reduce_parts<<<1, 1024, 0, st>>>(part_.get(), n_dec, C, g_wout);
     SGIPC_LAUNCH_CHECK();
     float* Gc = G_.get();
     float* Gn = G2_.get();
@@ -822,18 +859,17 @@ double Mpnn::loss_grad(hipStream_t st, const CoarseGraph& g, const float* X, con
         SGIPC_LAUNCH_CHECK();
         k_dw<<<n_dw, 256, 0, st>>>(rows, U_[l].get(), dY_.get(), part_.get());
         SGIPC_LAUNCH_CHECK();
-        k_reduce_parts<<<g256(2 * C * C), 256, 0, st>>>(part_.get(), n_dw, 2 * C * C,
-                                                         grad + 3 * C + (long)l * 2 * C * C);
+        k_reduce_parts<<<2 * C * C / 64, 1024, 0, st>>>(part_.get(), n_dw, 2 * C * C,
+                                                        grad + 3 * C + (long)l * 2 * C * C);
         SGIPC_LAUNCH_CHECK();
         if (l > 0) {
-            k_bwd_gather<<<gw, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), Gc, dU_.get(), Gn);
+            k_bwd_gather<<<gs, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), Gc, dU_.get(), Gn);
             SGIPC_LAUNCH_CHECK();
             std::swap(Gc, Gn);
         } else {
-            k_bwd_win<<<grid, 256, 0, st>>>(n, g.row_ptr.get(), g.col.get(), g.blk.get(), X, Gc, dU_.get(),
-                                            part_.get());
+            k_bwd_win<<<n_win, 256, 0, st>>>(rows, X, AX_.get(), Gc, dU_.get(), part_.get());
             SGIPC_LAUNCH_CHECK();
-            k_reduce_parts<<<1, 3 * C, 0, st>>>(part_.get(), n_win, 3 * C, g_win);
+            k_reduce_parts<<<3, 1024, 0, st>>>(part_.get(), n_win, 3 * C, g_win);
             SGIPC_LAUNCH_CHECK();
         }
     }

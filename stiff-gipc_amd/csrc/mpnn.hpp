@@ -88,6 +88,7 @@ class Mpnn {
     DevBuf<uint16_t> U_[kMpnnMaxLayers];
     DevBuf<float> Y_[kMpnnMaxLayers];
     DevBuf<float> G_, G2_, dU_, AV_;
+    DevBuf<float> AX_;      // Ahat X of the last training forward (3 columns)
     DevBuf<uint16_t> dY_;
     DevBuf<float> chat_, dchat_, part_;
     DevBuf<double> lpart_;
