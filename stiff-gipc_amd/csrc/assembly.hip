@@ -601,16 +601,407 @@ __global__ __launch_bounds__(256) void k_segment_sum(const double* __restrict__ 
     for (int q = 0; q < 9; ++q) o[q] = s[q];
 }
 
-__global__ void k_max_index(const int* __restrict__ rows, const int* __restrict__ cols, long n, int* __restrict__ out)
+// ------------------------------------------------------------------ conversion by rows
+// The general conversion above sorts 64-bit (row, column) keys over all their
+// bits, five passes over 16 M triplets at C1.  Triplets of one row are few (61
+// on average), so here they are put into row order by counting -- a
+// workgroup counts its rows in an LDS table, so memory sees one atomic per
+// distinct row and not one per triplet -- and each row is sorted by (column,
+// triplet) on its own: by one wave in registers up to 256 triplets, by one
+// workgroup in LDS up to 16384, and with a longer one the general conversion
+// runs instead.  The sums then read their triplets in exactly the general
+// order, 9 lanes per block (72-byte runs).  16 M triplets (1.47 GB in and
+// out): counting 81 + 103 us, row sorts 147, sums 440 (1.67 GB with the keys
+// at 3.8 TB/s; a large copy reaches 4.75 on this part), 0.9 ms with the index
+// check and the read-back against 1.73 ms for the general conversion.
+constexpr int kRowTable = 1024;  // slots of the LDS row table
+constexpr int kRowItems = 8;     // triplets per thread
+constexpr int kRowShort = 256, kRowMid = 2048, kRowLong = 16384;
+// words behind the row counts: bad index, a row past kRowLong, rows past
+// kRowShort, rows past kRowMid, unique blocks
+enum { kBad = 0, kTooLong, kNMid, kNLong, kUnique, kRowWords = 8 };
+
+// Counts of the rows (scatter = false), or the triplets' keys (column, then
+// index) to their row's segment (true; start: exclusive scan of the counts,
+// which are used up).  The order inside a segment is left to the row sort.
+template <bool scatter>
+__global__ __launch_bounds__(256) void k_rows_bin(const int* __restrict__ rows, const int* __restrict__ cols, long n,
+                                                  int n_rows, int* __restrict__ cnt, int* __restrict__ words,
+                                                  const int* __restrict__ start, uint64_t* __restrict__ key)
 {
-    int m = 0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        int r = rows[i], c = cols[i];
-        m = r > m ? r : m;
-        m = c > m ? c : m;
+    __shared__ int srow[kRowTable], scnt[kRowTable], sbase[kRowTable];
+    for (int i = threadIdx.x; i < kRowTable; i += 256) {
+        srow[i] = -1;
+        scnt[i] = 0;
     }
+    __syncthreads();
+    const long b0 = (long)blockIdx.x * (256 * kRowItems) + threadIdx.x;
+    int row[kRowItems], col[kRowItems], slot[kRowItems], at[kRowItems];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kRowItems; ++i) {
+        const long k = b0 + 256 * i;
+        row[i] = k < n ? rows[k] : -1;
+        col[i] = k < n ? cols[k] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < kRowItems; ++i) {
+        slot[i] = -1;
+        if (b0 + 256 * i >= n) continue;
+        if (row[i] < 0 || row[i] > col[i] || col[i] >= n_rows) {
+            bad = true;
+            row[i] = -1;
+            continue;
+        }
+        unsigned h = ((unsigned)row[i] * 2654435761u) >> 22;  // kRowTable slots
+        for (int t = 0; t < 6; ++t, h = (h + 1) & (kRowTable - 1)) {
+            const int r = atomicCAS(&srow[h], -1, row[i]);
+            if (r == -1 || r == row[i]) {
+                slot[i] = (int)h;
+                at[i] = atomicAdd(&scnt[h], 1);
+                break;
+            }
+        }
+    }
+    if (!scatter && bad) atomicOr(words + kBad, 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRowTable; i += 256)
+        if (scnt[i] > 0) {
+            if (scatter) sbase[i] = start[srow[i]] + atomicSub(cnt + srow[i], scnt[i]) - scnt[i];
+            else atomicAdd(cnt + srow[i], scnt[i]);
+        }
+    if (scatter) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kRowItems; ++i) {
+        if (row[i] < 0) continue;
+        if (scatter) {
+            const int p = slot[i] >= 0 ? sbase[slot[i]] + at[i] : start[row[i]] + atomicSub(cnt + row[i], 1) - 1;
+            key[p] = ((uint64_t)(uint32_t)col[i] << 32) | (uint32_t)(b0 + 256 * i);
+        } else if (slot[i] < 0) {
+            atomicAdd(cnt + row[i], 1);
+        }
+    }
+}
+
+// One wave per row: its keys sorted in place and its unique columns counted;
+// longer rows are listed.  Bitonic over 64 M elements, element i in lane
+// i % 64, register i / 64; the kernel is bound by its instructions (about 100
+// per row at M = 1; ranking every key against all others took 250, C1: 226
+// us against 147).
+template <int M>
+__device__ __forceinline__ int sort_row(uint64_t* __restrict__ seg, int k)
+{
+    const int lane = threadIdx.x & 63;
+    uint64_t v[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) v[m] = lane + 64 * m < k ? seg[lane + 64 * m] : ~0ull;
+#pragma unroll
+    for (int size = 2; size <= 64 * M; size <<= 1)
+#pragma unroll
+        for (int d = size >> 1; d > 0; d >>= 1) {
+            if (d >= 64) {
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const int q = m ^ (d / 64);
+                    if (q < m) continue;
+                    const bool up = ((64 * m) & size) == 0;
+                    const uint64_t x = v[m], y = v[q];
+                    const bool swap = (x > y) == up;
+                    v[m] = swap ? y : x;
+                    v[q] = swap ? x : y;
+                }
+            } else {
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const uint64_t x = v[m], y = __shfl_xor(x, d, 64);
+                    const bool up = ((64 * m + lane) & size) == 0, low = (lane & d) == 0;
+                    v[m] = (x < y) == (low == up) ? x : y;  // equal keys are all padding
+                }
+            }
+        }
+    int u = 0;
+    uint32_t before = 0;  // last column of the registers so far
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const uint32_t col = (uint32_t)(v[m] >> 32);
+        uint32_t prev = __shfl_up(col, 1, 64);
+        if (lane == 0) prev = before;
+        before = __shfl(col, 63, 64);
+        const bool in = lane + 64 * m < k;
+        if (in) seg[lane + 64 * m] = v[m];
+        u += __popcll(__ballot(in && ((m == 0 && lane == 0) || col != prev)));
+    }
+    return u;
+}
+__global__ __launch_bounds__(256) void k_rows_sort(int n_rows, const int* __restrict__ start, uint64_t* __restrict__ key,
+                                                   int* __restrict__ ucnt, int* __restrict__ words,
+                                                   int* __restrict__ list)
+{
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r > n_rows) return;
+    if (r == n_rows) {
+        if (lane == 0) ucnt[r] = 0;  // the scan's last element is the total
+        return;
+    }
+    const int b = start[r], k = start[r + 1] - b;
+    int u = 0;
+    if (k == 0) {
+    } else if (k <= 64) {
+        u = sort_row<1>(key + b, k);
+    } else if (k <= 128) {
+        u = sort_row<2>(key + b, k);
+    } else if (k <= kRowShort) {
+        u = sort_row<4>(key + b, k);
+    } else {
+        // listed from the front (up to kRowMid) or the back of the list
+        if (lane == 0) {
+            ucnt[r] = 0;  // until its own kernel sets it
+            if (k <= kRowMid) list[atomicAdd(words + kNMid, 1)] = r;
+            else list[n_rows - 1 - atomicAdd(words + kNLong, 1)] = r;
+            if (k > kRowLong) words[kTooLong] = 1;
+        }
+        return;
+    }
+    if (lane == 0) ucnt[r] = u;
+}
+
+// Longer rows, one workgroup each (a fixed grid walks the list): bitonic sort
+// in LDS, padded to a power of two.
+template <int CAP, int NT>
+__global__ __launch_bounds__(NT) void k_rows_sort_long(int n_rows, const int* __restrict__ start,
+                                                       uint64_t* __restrict__ key, int* __restrict__ ucnt,
+                                                       const int* __restrict__ words, const int* __restrict__ list)
+{
+    extern __shared__ uint64_t sk[];
+    __shared__ int su[NT / 64];
+    const int cnt = words[CAP == kRowMid ? kNMid : kNLong];
+    for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
+        const int r = list[CAP == kRowMid ? q : n_rows - 1 - q];
+        const int b = start[r], k = start[r + 1] - b;
+        if (k > CAP) continue;  // words[kTooLong]: the general conversion takes over
+        int p2 = 2 * kRowShort;
+        while (p2 < k) p2 <<= 1;
+        for (int i = threadIdx.x; i < p2; i += NT) sk[i] = i < k ? key[b + i] : ~0ull;
+        __syncthreads();
+        for (int size = 2; size <= p2; size <<= 1)
+            for (int d = size >> 1; d > 0; d >>= 1) {
+                for (int t = threadIdx.x; t < p2 / 2; t += NT) {
+                    const int i = 2 * t - (t & (d - 1)), j = i + d;
+                    const uint64_t x = sk[i], y = sk[j];
+                    if ((x > y) == ((i & size) == 0)) {
+                        sk[i] = y;
+                        sk[j] = x;
+                    }
+                }
+                __syncthreads();
+            }
+        int u = 0;
+        for (int i = threadIdx.x; i < k; i += NT) {
+            key[b + i] = sk[i];
+            u += (i == 0 || (sk[i - 1] >> 32) != (sk[i] >> 32)) ? 1 : 0;
+        }
+        u = wave_sum(u);
+        if ((threadIdx.x & 63) == 0) su[threadIdx.x >> 6] = u;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < NT / 64; ++w) u += su[w];
+            ucnt[r] = u;
+        }
+        __syncthreads();
+    }
+}
+
+// sum of value e of the triplets key[j0 .. j1) in order, four loads in flight
+__device__ __forceinline__ double sum_run(const double* __restrict__ tvals, const uint64_t* __restrict__ key, int j0,
+                                          int j1, int e)
+{
+    double s = 0.0;
+    int j = j0;
+    for (; j + 4 <= j1; j += 4) {
+        double v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = tvals[9 * (long)(uint32_t)key[j + t] + e];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s += v[t];
+    }
+    for (; j < j1; ++j) s += tvals[9 * (long)(uint32_t)key[j] + e];
+    return s;
+}
+
+// Unique blocks of the short rows, one wave per row, 9 lanes per block, 7
+// blocks at a time; a block of more than kSegChunk triplets is the ordered
+// sum of its chunk sums, as in the general conversion.
+__global__ __launch_bounds__(256) void k_rows_sum(const double* __restrict__ tvals, int n_rows,
+                                                  const int* __restrict__ start, const uint64_t* __restrict__ key,
+                                                  const int* __restrict__ uofs, int cap, double* __restrict__ ovals,
+                                                  int* __restrict__ orows, int* __restrict__ ocols,
+                                                  int* __restrict__ words)
+{
+    __shared__ uint64_t sm[4][kRowShort];
+    __shared__ int hd[4][kRowShort + 1];
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= n_rows) {
+        if (r == n_rows && lane == 0) words[kUnique] = uofs[n_rows];
+        return;
+    }
+    const int b = start[r], k = start[r + 1] - b;
+    if (k == 0 || k > kRowShort) return;
+    uint64_t* const sk = sm[threadIdx.x >> 6];
+    int* const h = hd[threadIdx.x >> 6];
+    const int o = uofs[r];
+    int u = 0, before = -1;  // last column of the previous 64
+    for (int i0 = 0; i0 < k; i0 += 64) {
+        const int i = i0 + lane;
+        const uint64_t w = i < k ? key[b + i] : 0ull;
+        const int col = (int)(w >> 32);
+        int prev = __shfl_up(col, 1, 64);
+        if (lane == 0) prev = before;
+        before = __shfl(col, 63, 64);
+        const bool head = i < k && col != prev;
+        const uint64_t m = __ballot(head);
+        if (i < k) sk[i] = w;
+        if (head) {
+            const int q = u + __popcll(m & ((1ull << lane) - 1ull));
+            h[q] = i;
+            if (o + q < cap) {
+                orows[o + q] = r;
+                ocols[o + q] = col;
+            }
+        }
+        u += __popcll(m);
+    }
+    if (lane == 0) h[u] = k;
+    wave_lds_sync();
+    const int g = lane / 9, e = lane % 9;
+    if (g == 7) return;
+    for (int q = g; q < u; q += 7) {
+        const int j0 = h[q], j1 = h[q + 1];
+        double s = 0.0;
+        if (j1 - j0 <= kSegChunk) {
+            s = sum_run(tvals, sk, j0, j1, e);
+        } else {
+            for (int c = j0; c < j1; c += kSegChunk) s += sum_run(tvals, sk, c, min(c + kSegChunk, j1), e);
+        }
+        if (o + q < cap) ovals[9 * (long)(o + q) + e] = s;
+    }
+}
+
+// Unique blocks of the longer rows, one workgroup per row: the 9-lane groups
+// of all waves take the blocks' chunks in turn (blocks without chunks count
+// as one), then the chunk sums of each block are added in order.
+template <int CAP, int NT>
+__global__ __launch_bounds__(NT) void k_rows_sum_long(const double* __restrict__ tvals, int n_rows,
+                                                      const int* __restrict__ start, const uint64_t* __restrict__ key,
+                                                      const int* __restrict__ uofs, int cap,
+                                                      double* __restrict__ ovals, int* __restrict__ orows,
+                                                      int* __restrict__ ocols, const int* __restrict__ words,
+                                                      const int* __restrict__ list)
+{
+    // chunk sums of the blocks past kSegChunk: their count is below 2 CAP / kSegChunk
+    extern __shared__ double part[];
+    __shared__ int wsum[NT / 64], wblk[NT / 64];
+    constexpr int kGroups = 7 * (NT / 64);
+    const int cnt = words[CAP == kRowMid ? kNMid : kNLong];
+    int* const head = reinterpret_cast<int*>(part + 9 * (2 * CAP / kSegChunk));  // CAP + 1 block starts
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int t = blockIdx.x; t < cnt; t += gridDim.x) {
+        const int r = list[CAP == kRowMid ? t : n_rows - 1 - t];
+        const int b = start[r], k = start[r + 1] - b, o = uofs[r];
+        if (k > CAP) continue;
+        // block starts in order
+        int u = 0;
+        for (int i0 = 0; i0 < k; i0 += NT) {
+            const int i = i0 + (int)threadIdx.x;
+            const uint64_t w = i < k ? key[b + i] : 0ull;
+            const bool hdf = i < k && (i == 0 || (key[b + i - 1] >> 32) != (w >> 32));
+            const uint64_t m = __ballot(hdf);
+            if (lane == 0) wsum[wv] = __popcll(m);
+            __syncthreads();
+            int before = u, all = 0;
+            for (int q = 0; q < NT / 64; ++q) {
+                if (q < wv) before += wsum[q];
+                all += wsum[q];
+            }
+            if (hdf) {
+                const int q = before + __popcll(m & ((1ull << lane) - 1ull));
+                head[q] = i;
+                if (o + q < cap) {
+                    orows[o + q] = r;
+                    ocols[o + q] = (int)(w >> 32);
+                }
+            }
+            u += all;
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) head[u] = k;
+        __syncthreads();
+        const int g = wv * 7 + lane / 9, e = lane % 9;
+        const bool use = lane < 63;
+        // blocks of at most kSegChunk triplets, and the chunks of the others
+        int some = 0;
+        for (int q = g; q < u && use; q += kGroups) {
+            const int j0 = head[q], j1 = head[q + 1];
+            if (j1 - j0 > kSegChunk) {
+                some = 1;
+                continue;
+            }
+            const double s = sum_run(tvals, key + b, j0, j1, e);
+            if (o + q < cap) ovals[9 * (long)(o + q) + e] = s;
+        }
+        if (__syncthreads_or(some) == 0) continue;
+        int c = 0;  // chunks so far; every lane walks the blocks
+        for (int q = 0; q < u; ++q) {
+            const int j0 = head[q], j1 = head[q + 1];
+            if (j1 - j0 <= kSegChunk) continue;
+            const int nc = (j1 - j0 + kSegChunk - 1) / kSegChunk;
+            // the group that takes chunk x is x % kGroups
+            for (int x = c + (g - c % kGroups + kGroups) % kGroups; x < c + nc && use; x += kGroups) {
+                const int f = j0 + (x - c) * kSegChunk;
+                part[9 * x + e] = sum_run(tvals, key + b, f, min(f + kSegChunk, j1), e);
+            }
+            c += nc;
+        }
+        __syncthreads();
+        c = 0;
+        for (int q = 0, nl = 0; q < u; ++q) {
+            const int j0 = head[q], j1 = head[q + 1];
+            if (j1 - j0 <= kSegChunk) continue;
+            const int nc = (j1 - j0 + kSegChunk - 1) / kSegChunk;
+            if (nl++ % kGroups == g && use) {
+                double s = 0.0;
+                for (int x = c; x < c + nc; ++x) s += part[9 * x + e];
+                if (o + q < cap) ovals[9 * (long)(o + q) + e] = s;
+            }
+            c += nc;
+        }
+        __syncthreads();
+    }
+}
+
+// One atomic per workgroup (at most 512): a wave's atomic each, 1024 of them
+// on one address, took longer than the 128 MB of C1's indices.
+__global__ __launch_bounds__(256) void k_max_index(const int* __restrict__ rows, const int* __restrict__ cols, long n,
+                                                   int* __restrict__ out)
+{
+    __shared__ int sm[4];
+    int m = 0;
+    const long stride = (long)gridDim.x * blockDim.x;
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        int v[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[2 * k] = rows[i + k * stride];
+            v[2 * k + 1] = cols[i + k * stride];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) m = max(m, v[k]);
+    }
+    for (; i < n; i += stride) m = max(m, max(rows[i], cols[i]));
     m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(out, max(max(sm[0], sm[1]), max(sm[2], sm[3])));
 }
 
 inline int g256(long n) { return (int)((n + 255) / 256); }
@@ -648,7 +1039,7 @@ void launch_mass_diag(hipStream_t s, int n, const double* mass, int hess_offset,
 int convert_max_index(hipStream_t s, const int* rows, const int* cols, long n, int* ints)
 {
     launch_fill<int>(s, ints, 0, 1);
-    k_max_index<<<256, 256, 0, s>>>(rows, cols, n, ints);
+    k_max_index<<<(int)std::min<long>(512, g256(n)), 256, 0, s>>>(rows, cols, n, ints);
     SGIPC_LAUNCH_CHECK();
     int m = 0;
     SGIPC_HIP(hipMemcpyAsync(&m, ints, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -737,11 +1128,89 @@ int Converter::max_index(hipStream_t s, const int* rows, const int* cols, long n
     return convert_max_index(s, rows, cols, n, scratch_int_.get());
 }
 
+bool Converter::convert_rows(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n,
+                             int n_rows, double* ovals, int* orows, int* ocols, int capacity, int* unique)
+{
+    const long R = n_rows;
+    row_cnt_.reserve(R + 1 + kRowWords);
+    row_start_.reserve(R + 1);
+    row_ucnt_.reserve(R + 1);
+    row_uofs_.reserve(R + 1);
+    row_list_.reserve(R > 0 ? R : 1);
+    keys_.reserve(n);
+    int* const cnt = row_cnt_.get();
+    int* const words = cnt + R + 1;
+    size_t need = 0;
+    SGIPC_HIP(rocprim::exclusive_scan(nullptr, need, cnt, row_start_.get(), 0, (size_t)(R + 1), rocprim::plus<int>(), s));
+    temp_.reserve(need);
+    launch_fill<int>(s, cnt, 0, R + 1 + kRowWords);
+    const int gb = (int)((n + 256 * kRowItems - 1) / (256 * kRowItems));
+    k_rows_bin<false><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, nullptr, nullptr);
+    SGIPC_LAUNCH_CHECK();
+    SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, cnt, row_start_.get(), 0, (size_t)(R + 1),
+                                      rocprim::plus<int>(), s));
+    k_rows_bin<true><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, row_start_.get(), keys_.get());
+    SGIPC_LAUNCH_CHECK();
+    const int gr = (int)((R + 1 + 3) / 4);
+    k_rows_sort<<<gr, 256, 0, s>>>(n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+    SGIPC_LAUNCH_CHECK();
+    // the longer rows: grids that walk the lists (their lengths stay on the device)
+    const int g_mid = (int)std::min<long>(1024, n / kRowShort), g_long = (int)std::min<long>(256, n / kRowMid);
+    if (g_mid > 0) {
+        k_rows_sort_long<kRowMid, 256><<<g_mid, 256, kRowMid * sizeof(uint64_t), s>>>(
+            n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+        SGIPC_LAUNCH_CHECK();
+    }
+    auto sum_lds = [](int cap) { return 9 * sizeof(double) * (2 * cap / kSegChunk) + sizeof(int) * (cap + 1); };
+    if (g_long > 0) {
+        // more LDS than a launch gets by default (set on the current device)
+        SGIPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rows_sort_long<kRowLong, 1024>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, kRowLong * sizeof(uint64_t)));
+        SGIPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rows_sum_long<kRowLong, 1024>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds(kRowLong)));
+        k_rows_sort_long<kRowLong, 1024><<<g_long, 1024, kRowLong * sizeof(uint64_t), s>>>(
+            n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+        SGIPC_LAUNCH_CHECK();
+    }
+    SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, row_ucnt_.get(), row_uofs_.get(), 0, (size_t)(R + 1),
+                                      rocprim::plus<int>(), s));
+    k_rows_sum<<<gr, 256, 0, s>>>(tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals,
+                                  orows, ocols, words);
+    SGIPC_LAUNCH_CHECK();
+    if (g_mid > 0) {
+        k_rows_sum_long<kRowMid, 256><<<g_mid, 256, sum_lds(kRowMid), s>>>(
+            tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals, orows, ocols, words,
+            row_list_.get());
+        SGIPC_LAUNCH_CHECK();
+    }
+    if (g_long > 0) {
+        k_rows_sum_long<kRowLong, 1024><<<g_long, 1024, sum_lds(kRowLong), s>>>(
+            tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals, orows, ocols, words,
+            row_list_.get());
+        SGIPC_LAUNCH_CHECK();
+    }
+    int h[kRowWords];
+    SGIPC_HIP(hipMemcpyAsync(h, words, sizeof(h), hipMemcpyDeviceToHost, s));
+    SGIPC_HIP(hipStreamSynchronize(s));
+    SGIPC_CHECK(h[kBad] == 0, SGIPC_BAD_INDEX,
+                "triplet with row > col, a negative index or an index beyond the bound");
+    if (h[kTooLong]) return false;
+    *unique = h[kUnique];
+    SGIPC_CHECK(*unique <= capacity, SGIPC_CAPACITY, "unique block count exceeds the output capacity");
+    return true;
+}
+
 int Converter::convert(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n,
                        int index_bound, double* ovals, int* orows, int* ocols, int capacity)
 {
     if (n <= 0) return 0;
     SGIPC_CHECK(n < (1L << 31), SGIPC_CAPACITY, "too many triplets");
+    // By rows unless the rows are so few that they must be long (then their
+    // sorts would leave the chip idle), or so many that their tables outweigh
+    // the triplets, or one proves too long.
+    if (index_bound < (1L << 31) - 8 && n <= 2048L * index_bound && index_bound <= 4 * n + 4096 &&
+        convert_rows(s, tvals, trows, tcols, n, index_bound, ovals, orows, ocols, capacity, &last_unique))
+        return last_unique;
     keys_.reserve(n);
     skeys_.reserve(n);
     idx_.reserve(n);

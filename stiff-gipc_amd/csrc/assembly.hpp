@@ -62,6 +62,11 @@ class Converter {
     int last_unique = 0;
 
   private:
+    // The conversion by row counting and per-row sorts; false when a row is
+    // too long for it (nothing of use written then).
+    bool convert_rows(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n, int n_rows,
+                      double* ovals, int* orows, int* ocols, int capacity, int* unique);
+    DevBuf<int> row_cnt_, row_start_, row_ucnt_, row_uofs_, row_list_;
     DevBuf<uint64_t> keys_, skeys_;
     DevBuf<int> idx_, sidx_, flag_, pos_, head_, scratch_int_;
     DevBuf<unsigned char> temp_;

@@ -125,16 +125,6 @@ __global__ void k_g_blocks(const uint64_t* __restrict__ sk, const int* __restric
 }
 
 // ------------------------------------------------------------------ layers
-// Workgroup b of the n workgroups of a gather -> its place in the order
-// (sample, node): the 8 XCDs take workgroups in turn, so XCD b % 8 gets one
-// contiguous run, i.e. whole samples or stretches of neighbouring nodes whose
-// rows its own L2 then holds (a sample's 64 channels are 6 MB at 8k nodes).
-__device__ __forceinline__ int xcd_run(int b, int n)
-{
-    const int x = b & 7, q = n >> 3, r = n & 7;
-    return x * q + (x < r ? x : r) + (b >> 3);
-}
-
 // sum over node i's row of Ahat_ij (3 x 64 rows of src at row stride ld):
 // 16 lanes take 4 channels each, the wave's 4 groups every fourth neighbour
 // (4 load chains in flight); the groups are added in a fixed order and every
@@ -171,7 +161,9 @@ __device__ __forceinline__ void gather64(const int* __restrict__ rp, const int* 
         }
 }
 
-// Y = Ahat V on 64 channels: one wave per node of every sample.
+// Y = Ahat V on 64 channels: one wave per node of every sample; each XCD
+// takes whole samples or stretches of neighbouring nodes (xcd_run), whose rows
+// its own L2 then holds (a sample's 64 channels are 6 MB at 8k nodes).
 __global__ __launch_bounds__(256) void k_spmm64(int n, const int* __restrict__ rp, const int* __restrict__ colx,
                                                 const float* __restrict__ blk, const float* __restrict__ V,
                                                 float* __restrict__ Y)

@@ -35,6 +35,15 @@ __device__ __forceinline__ T wave_max(T v)
     return v;
 }
 
+// Workgroup b of n -> its place in a contiguous run per XCD: the 8 XCDs take
+// workgroups in turn, so XCD b % 8 gets run [x n / 8 ..) and its L2 holds what
+// neighbours share.  A bijection on [0, n).
+__device__ __forceinline__ int xcd_run(int b, int n)
+{
+    const int x = b & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (b >> 3);
+}
+
 // Index of the highest set bit of m that is <= lane (m must have one such bit).
 __device__ __forceinline__ int seg_start_from_heads(uint64_t heads, int lane)
 {
