@@ -333,7 +333,7 @@ int sgipc_spmat_apply_f32_values(sgipc_spmat* m, double a, const double* x, doub
  * column words index each tile's LDS copy of x (own rows + halo), 0 for the
  * global-gather form (taken when that copy does not fit in LDS, or when the
  * environment variable SGIPC_SPMV_GATHER is set to a non-zero value at
- * create()); *halo_max = largest halo of a 512-row tile (vertices);
+ * create()); *halo_max = largest halo of a row tile (vertices);
  * *tl_slots = in-tile transposed slots the fullest tile uses.  Any output
  * pointer may be NULL. */
 int sgipc_spmat_layout(const sgipc_spmat* m, int* halo_form, int* halo_max, int* tl_slots);

@@ -5,7 +5,7 @@
 // Here the matrix is re-laid out once per Newton step so that each upper
 // block is read from HBM once per SpMV without atomics:
 //
-//   * rows are cut into tiles of kTile consecutive (Morton-ordered) rows; one
+//   * rows are cut into tiles of 64, 128 or 512 consecutive (Morton-ordered) rows; one
 //     workgroup owns a tile and writes every row of it exactly once;
 //   * an upper block (i, j) with both ends in the same tile is stored once, in
 //     row i.  Its H x_j goes to row i in registers, its H^T x_i to a slot of
@@ -48,33 +48,28 @@ namespace sgipc {
 
 namespace {
 
-constexpr int kTile = 512;                 // rows per workgroup
-constexpr int kSplit = 2;                  // waves per slice
-constexpr int kThreads = kTile * kSplit;   // 1024
+// Rows per workgroup.  Large tiles hold more blocks in their tile (stored
+// once) and gather smaller halos, small ones give matrices of few rows enough
+// workgroups: back to back, FP64 / FP32 values, us per product of a
+// 27-neighbour grid with contacts at 4k, 32k, 64k, 110k and 262k rows
+//   512 rows   13.5 / 10.8   16.0 / 11.5   17.2 / 12.3   19.4 / 13.9   43.8 / 24.8
+//   128 rows    8.1 /  7.3    9.7 /  8.1   13.7 / 10.0   22.7 / 18.2   49.7 / 39.2
+//    64 rows    7.1 /  6.5    9.8 /  7.6   18.4 / 14.7   27.1 / 25.5   62.2 / 56.0
+constexpr int kTileLarge = 512, kTileMid = 128, kTileSmall = 64;
+// up to 512 rows one tile holds the whole matrix (no halo); below these counts
+// the smaller tiles
+constexpr int kRowsSmall = 28000, kRowsMid = 80000;
+constexpr int kSplit = 2;                  // waves per slice (gather form)
 constexpr int kTcap = 4096;                // in-tile transposed slots per tile (LDS)
 constexpr uint32_t kInTile = 0x80000000u;
-constexpr int kWaves = kThreads / 64;          // waves of a workgroup
-constexpr int kSlices = kTile / 64;            // SELL-64 slices of a tile
-constexpr int kPieces = kWaves + kSlices - 1;  // (wave, slice) partial rows of the halo kernel
 constexpr int kLdsBytes = 163840;              // LDS of one CU on gfx950
 constexpr int kLongRow = 128;                  // rows with more blocks are kept outside the tiles
-
-// Workgroups are handed to the 8 XCDs of the part round-robin in blockIdx
-// order.  Mapping block b to tile start(b % 8) + b / 8 gives every XCD a
-// contiguous run of tiles, so the x entries neighbouring tiles share are
-// fetched into one XCD's L2 instead of into all of them.  A bijection on
-// [0, n): XCD x owns n / 8 + (x < n % 8) tiles starting at x (n / 8) + min(x, n % 8).
-__device__ __forceinline__ int xcd_tile(int b, int n)
-{
-    const int x = b & 7, q = n >> 3, rem = n & 7;
-    return x * q + (x < rem ? x : rem) + (b >> 3);
-}
 
 // With kFuseP the gathered vector is p_new = z + beta p_old, formed on the fly
 // (beta = rz_new / rz_old from partials, summed in a fixed order), and every
 // owned row of p_new is written: the PCG p update rides along with the SpMV.
-template <typename TM, typename TV, bool kDot, bool kFuseP>
-__global__ __launch_bounds__(kThreads) void k_spmv_tsym(const TM* __restrict__ vals, const uint32_t* __restrict__ cw,
+template <typename TM, typename TV, int kTile, bool kDot, bool kFuseP>
+__global__ __launch_bounds__(kTile * kSplit) void k_spmv_tsym(const TM* __restrict__ vals, const uint32_t* __restrict__ cw,
                                                         const int* __restrict__ slice_ptr,
                                                         const int* __restrict__ slice_w, const int* __restrict__ perm,
                                                         const int* __restrict__ plen,
@@ -85,6 +80,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv_tsym(const TM* __restrict__ v
                                                         const double* __restrict__ rzn,
                                                         const double* __restrict__ rzo, int n_rz, int n_rows)
 {
+    constexpr int kThreads = kTile * kSplit;
     __shared__ TV tl[kTcap * 3];
     __shared__ TV red[3 * kTile];
     __shared__ TV xs[3 * kTile];  // the gathered vector over this tile's own rows
@@ -98,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void k_spmv_tsym(const TM* __restrict__ v
         if (kFuseP) return (TV)((double)zf[k] + beta * (double)x[k]);
         return x[k];
     };
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = xcd_run(blockIdx.x, gridDim.x);
     {
         // in-tile columns read x from LDS: one coalesced load of the tile's rows
         const long b3 = 3L * tile * kTile, e3 = 3L * n_rows;
@@ -234,24 +230,14 @@ __global__ __launch_bounds__(kThreads) void k_spmv_tsym(const TM* __restrict__ v
 // in the vector type) in 512-thread workgroups, two of which fit a CU's LDS
 // and registers, so one workgroup's staging and reduction overlap the other's
 // stream.
-template <typename TM, typename TV>
+template <typename TM, typename TV, int kTile>
 struct HaloCfg {
-    static constexpr int NT = 1024;
-    using TL = TV;
-};
-template <>
-struct HaloCfg<float, double> {
-    static constexpr int NT = 512;
-    using TL = float;
-};
-template <>
-struct HaloCfg<float, float> {
-    static constexpr int NT = 512;
-    using TL = float;
+    static constexpr int NT = kTile == kTileLarge && sizeof(TM) == 8 ? 1024 : 512;
+    using TL = typename std::conditional<sizeof(TM) == 4, float, TV>::type;
 };
 
-template <typename TM, typename TV, bool kDot, bool kFuseP, bool kSum1 = false>
-__global__ __launch_bounds__((HaloCfg<TM, TV>::NT), 4) void k_spmv_halo(const TM* __restrict__ vals, const uint32_t* __restrict__ cw,
+template <typename TM, typename TV, int kTile, bool kDot, bool kFuseP, bool kSum1 = false>
+__global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(const TM* __restrict__ vals, const uint32_t* __restrict__ cw,
                                                         const int* __restrict__ slice_ptr,
                                                         const int* __restrict__ perm, const int* __restrict__ plen,
                                                         const uint32_t* __restrict__ tinfo,
@@ -265,9 +251,10 @@ __global__ __launch_bounds__((HaloCfg<TM, TV>::NT), 4) void k_spmv_halo(const TM
                                                         const double* __restrict__ rzo, int n_rz, int n_rows,
                                                         Level1Sums l1)
 {
-    using TL = typename HaloCfg<TM, TV>::TL;
-    constexpr int kThreads = HaloCfg<TM, TV>::NT;
+    using TL = typename HaloCfg<TM, TV, kTile>::TL;
+    constexpr int kThreads = HaloCfg<TM, TV, kTile>::NT;
     constexpr int kWaves = kThreads / 64;
+    constexpr int kSlices = kTile / 64;
     constexpr int kPieces = kWaves + kSlices - 1;
     constexpr bool kExactLds = std::is_same<TL, TV>::value;
     extern __shared__ __align__(16) unsigned char lds_dyn[];
@@ -287,7 +274,7 @@ __global__ __launch_bounds__((HaloCfg<TM, TV>::NT), 4) void k_spmv_halo(const TM
         if (kFuseP) return (TV)((double)zf[k] + beta * (double)x[k]);
         return x[k];
     };
-    const int tile = order[xcd_tile(blockIdx.x, gridDim.x)];
+    const int tile = order[xcd_run(blockIdx.x, gridDim.x)];
     const long b3 = 3L * tile * kTile;
     const int q0 = tile * kSlices;
     const long A = slice_ptr[q0];
@@ -588,7 +575,7 @@ __global__ void k_long_flags(const int* __restrict__ up_ptr, const int* __restri
 }
 
 // in-tile candidate flag per col-sorted entry (i != j, same tile, neither row long)
-__global__ void k_cand(const uint64_t* __restrict__ skeys, int nnz, int kbits, const int* __restrict__ lflag,
+__global__ void k_cand(int tile_rows, const uint64_t* __restrict__ skeys, int nnz, int kbits, const int* __restrict__ lflag,
                        int* __restrict__ cand)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -596,7 +583,7 @@ __global__ void k_cand(const uint64_t* __restrict__ skeys, int nnz, int kbits, c
     const uint64_t key = skeys[s];
     const int j = (int)(key >> kbits);
     const int i = (int)(key & ((1ull << kbits) - 1ull));
-    cand[s] = (i != j && i / kTile == j / kTile && !lflag[i] && !lflag[j]) ? 1 : 0;
+    cand[s] = (i != j && i / tile_rows == j / tile_rows && !lflag[i] && !lflag[j]) ? 1 : 0;
 }
 
 // Rank -> row of the long rows and their CSR starts (one thread per row;
@@ -692,14 +679,14 @@ __global__ __launch_bounds__(256) void k_spmv_long(const int* __restrict__ long_
 // Per column j: the upper word of every block (i, j), the in-tile slot range of
 // column j and the count of lower (cross-tile) entries row j stores.
 // A candidate whose rank in its tile reaches kTcap is stored as cross-tile.
-__global__ void k_col_words(const uint64_t* __restrict__ skeys, const int* __restrict__ sidx,
+__global__ void k_col_words(int tile_rows, const uint64_t* __restrict__ skeys, const int* __restrict__ sidx,
                             const int* __restrict__ cscan, const int* __restrict__ col_ptr, int n, int kbits,
                             const int* __restrict__ lflag, uint32_t* __restrict__ up_word,
                             uint32_t* __restrict__ tinfo, int* __restrict__ low_cnt)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
-    const int tile0 = (j / kTile) * kTile;
+    const int tile0 = (j / tile_rows) * tile_rows;
     const int rank_base = cscan[col_ptr[tile0]];
     int tb = -1, tcount = 0, low = 0;
     for (int s = col_ptr[j]; s < col_ptr[j + 1]; ++s) {
@@ -709,7 +696,7 @@ __global__ void k_col_words(const uint64_t* __restrict__ skeys, const int* __res
             up_word[b] = (uint32_t)j;
             continue;
         }
-        const bool same = i / kTile == j / kTile;
+        const bool same = i / tile_rows == j / tile_rows;
         const int rank = cscan[s] - rank_base;
         if (same && !lflag[i] && !lflag[j] && rank < kTcap) {
             up_word[b] = kInTile | ((uint32_t)(j - tile0) << 16) | (uint32_t)rank;
@@ -725,7 +712,7 @@ __global__ void k_col_words(const uint64_t* __restrict__ skeys, const int* __res
     low_cnt[j] = low;
 }
 
-__global__ void k_row_keys(const int* __restrict__ up_ptr, const int* __restrict__ low_cnt,
+__global__ void k_row_keys(int tile_rows, const int* __restrict__ up_ptr, const int* __restrict__ low_cnt,
                            const int* __restrict__ lflag, int n, int* __restrict__ len, uint64_t* __restrict__ key,
                            int* __restrict__ iota)
 {
@@ -733,7 +720,7 @@ __global__ void k_row_keys(const int* __restrict__ up_ptr, const int* __restrict
     if (i >= n) return;
     const int L = lflag[i] ? 0 : (up_ptr[i + 1] - up_ptr[i]) + low_cnt[i];
     len[i] = L;
-    key[i] = ((uint64_t)(i / kTile) << 16) | (uint64_t)(0xFFFFu - (uint32_t)(L < 0xFFFF ? L : 0xFFFF));
+    key[i] = ((uint64_t)(i / tile_rows) << 16) | (uint64_t)(0xFFFFu - (uint32_t)(L < 0xFFFF ? L : 0xFFFF));
     iota[i] = i;
 }
 
@@ -852,7 +839,7 @@ __global__ __launch_bounds__(256) void k_pack(const double* __restrict__ vals, c
 // A word that is not an in-tile transposed slot names a global column; it is
 // external when the column lies outside the slot's tile.  Padding rows are
 // skipped (their words are rewritten to local index 0 and never used).
-__global__ void k_ext_count(const uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
+__global__ void k_ext_count(int tile_rows, const uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
                             const int* __restrict__ perm, int n_slices, int* __restrict__ cnt)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -860,27 +847,27 @@ __global__ void k_ext_count(const uint32_t* __restrict__ cw, const int* __restri
     const int q = t >> 6, lane = t & 63;
     int c = 0;
     if (perm[t] >= 0) {
-        const int tile = q / kSlices;
+        const int tile = q / (tile_rows / 64);
         for (long s = slice_ptr[q]; s < slice_ptr[q + 1]; ++s) {
             const uint32_t w = cw[s * 64 + lane];
-            if (!(w & kInTile) && (int)w / kTile != tile) ++c;
+            if (!(w & kInTile) && (int)w / tile_rows != tile) ++c;
         }
     }
     cnt[t] = c;
 }
 
-__global__ void k_ext_emit(const uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
+__global__ void k_ext_emit(int tile_rows, const uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
                            const int* __restrict__ perm, const int* __restrict__ off, int n_slices,
                            uint64_t* __restrict__ keys)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_slices * 64 || perm[t] < 0) return;
     const int q = t >> 6, lane = t & 63;
-    const int tile = q / kSlices;
+    const int tile = q / (tile_rows / 64);
     int o = off[t];
     for (long s = slice_ptr[q]; s < slice_ptr[q + 1]; ++s) {
         const uint32_t w = cw[s * 64 + lane];
-        if (!(w & kInTile) && (int)w / kTile != tile) keys[o++] = ((uint64_t)tile << 32) | (uint64_t)w;
+        if (!(w & kInTile) && (int)w / tile_rows != tile) keys[o++] = ((uint64_t)tile << 32) | (uint64_t)w;
     }
 }
 
@@ -931,15 +918,15 @@ __global__ void k_tile_stats(const int* __restrict__ halo_ptr, const uint32_t* _
 }
 
 // rewrite the words as local indices: own rows (column - tile start), halo
-// vertices (kTile + rank in the tile's ascending halo list)
-__global__ void k_localize(uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
+// vertices (tile_rows + rank in the tile's ascending halo list)
+__global__ void k_localize(int tile_rows, uint32_t* __restrict__ cw, const int* __restrict__ slice_ptr,
                            const int* __restrict__ perm, const int* __restrict__ halo_ptr,
                            const int* __restrict__ halo_list, int n_slices)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_slices * 64) return;
     const int q = t >> 6, lane = t & 63;
-    const int tile = q / kSlices;
+    const int tile = q / (tile_rows / 64);
     const bool pad = perm[t] < 0;
     const int h0 = halo_ptr[tile], h1 = halo_ptr[tile + 1];
     for (long s = slice_ptr[q]; s < slice_ptr[q + 1]; ++s) {
@@ -948,15 +935,15 @@ __global__ void k_localize(uint32_t* __restrict__ cw, const int* __restrict__ sl
         uint32_t lw = 0;
         if (!pad) {
             const int j = (int)w;
-            if (j / kTile == tile) {
-                lw = (uint32_t)(j - tile * kTile) << 16;
+            if (j / tile_rows == tile) {
+                lw = (uint32_t)(j - tile * tile_rows) << 16;
             } else {
                 int lo = h0, hi = h1;
                 while (lo < hi) {
                     const int mid = (lo + hi) >> 1;
                     if (halo_list[mid] < j) lo = mid + 1; else hi = mid;
                 }
-                lw = (uint32_t)(kTile + (lo - h0)) << 16;
+                lw = (uint32_t)(tile_rows + (lo - h0)) << 16;
             }
         }
         cw[s * 64 + lane] = lw;
@@ -986,8 +973,9 @@ void FullMatrix::build(hipStream_t s, const double* vals, const int* rows, const
     has_f32 = want_f32;
     int kbits = 1;
     while (kbits < 31 && (1L << kbits) < (long)n) ++kbits;
-    n_tiles = (n + kTile - 1) / kTile;
-    const int n_pos = n_tiles * kTile;
+    tile_rows = n <= kTileLarge ? kTileLarge : n < kRowsSmall ? kTileSmall : (n < kRowsMid ? kTileMid : kTileLarge);
+    n_tiles = (n + tile_rows - 1) / tile_rows;
+    const int n_pos = n_tiles * tile_rows;
     n_slices = n_pos / 64;
     keys_.reserve(nnz_up);
     skeys_.reserve(nnz_up);
@@ -1051,16 +1039,16 @@ void FullMatrix::build(hipStream_t s, const double* vals, const int* rows, const
     SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need5, llen_.get(), loff_.get(), 0, (size_t)n + 1,
                                       rocprim::plus<int>(), s));
     // in-tile ranks: exclusive scan of the candidate flags in column order
-    k_cand<<<g256(nnz_up), 256, 0, s>>>(skeys_.get(), nnz_up, kbits, lflag_.get(), cand_.get());
+    k_cand<<<g256(nnz_up), 256, 0, s>>>(tile_rows, skeys_.get(), nnz_up, kbits, lflag_.get(), cand_.get());
     SGIPC_LAUNCH_CHECK();
     SGIPC_HIP(hipMemsetAsync(cand_.get() + nnz_up, 0, sizeof(int), s));
     SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need2, cand_.get(), cscan_.get(), 0, (size_t)nnz_up + 1,
                                       rocprim::plus<int>(), s));
-    k_col_words<<<g256(n), 256, 0, s>>>(skeys_.get(), sidx_.get(), cscan_.get(), col_ptr_.get(), n, kbits,
+    k_col_words<<<g256(n), 256, 0, s>>>(tile_rows, skeys_.get(), sidx_.get(), cscan_.get(), col_ptr_.get(), n, kbits,
                                         lflag_.get(), up_word_.get(), tinfo.get(), low_cnt_.get());
     SGIPC_LAUNCH_CHECK();
     // rows sorted by entry count inside each tile
-    k_row_keys<<<g256(n), 256, 0, s>>>(up_ptr_.get(), low_cnt_.get(), lflag_.get(), n, len_.get(), rkey_.get(),
+    k_row_keys<<<g256(n), 256, 0, s>>>(tile_rows, up_ptr_.get(), low_cnt_.get(), lflag_.get(), n, len_.get(), rkey_.get(),
                                        iota_.get());
     SGIPC_LAUNCH_CHECK();
     SGIPC_HIP(rocprim::radix_sort_pairs(temp_.get(), need3, rkey_.get(), rkey_sorted_.get(), iota_.get(),
@@ -1121,7 +1109,7 @@ void FullMatrix::build_halo(hipStream_t s, int tbits)
     SGIPC_HIP(rocprim::exclusive_scan(nullptr, need, hcnt_.get(), hoff_.get(), 0, (size_t)nl + 1, rocprim::plus<int>(),
                                       s));
     temp_.reserve(need);
-    k_ext_count<<<g256(nl), 256, 0, s>>>(sell_cols.get(), slice_ptr.get(), perm.get(), n_slices, hcnt_.get());
+    k_ext_count<<<g256(nl), 256, 0, s>>>(tile_rows, sell_cols.get(), slice_ptr.get(), perm.get(), n_slices, hcnt_.get());
     SGIPC_LAUNCH_CHECK();
     SGIPC_HIP(hipMemsetAsync(hcnt_.get() + nl, 0, sizeof(int), s));
     SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, hcnt_.get(), hoff_.get(), 0, (size_t)nl + 1,
@@ -1142,7 +1130,7 @@ void FullMatrix::build_halo(hipStream_t s, int tbits)
         SGIPC_HIP(rocprim::inclusive_scan(nullptr, n2, hflag_.get(), hinc_.get(), (size_t)n_ext, rocprim::plus<int>(),
                                           s));
         temp_.reserve(n1 > n2 ? n1 : n2);
-        k_ext_emit<<<g256(nl), 256, 0, s>>>(sell_cols.get(), slice_ptr.get(), perm.get(), hoff_.get(), n_slices,
+        k_ext_emit<<<g256(nl), 256, 0, s>>>(tile_rows, sell_cols.get(), slice_ptr.get(), perm.get(), hoff_.get(), n_slices,
                                             hkeys_.get());
         SGIPC_LAUNCH_CHECK();
         SGIPC_HIP(rocprim::radix_sort_keys(temp_.get(), n1, hkeys_.get(), hkeys_sorted_.get(), (size_t)n_ext, 0,
@@ -1172,21 +1160,23 @@ void FullMatrix::build_halo(hipStream_t s, int tbits)
     tl_max = st[1] > 0 ? st[1] : 1;
     // the FP64-vector kernels have the largest LDS; use the halo form only when
     // it fits beside the largest static LDS among them
-    if (halo_dyn_bytes(sizeof(double), kThreads) + halo_static_lds() > (size_t)kLdsBytes) return;
+    const int threads = tile_rows == kTileLarge ? HaloCfg<double, double, kTileLarge>::NT
+                                                : HaloCfg<double, double, kTileSmall>::NT;
+    if (halo_dyn_bytes(sizeof(double), threads) + halo_static_lds() > (size_t)kLdsBytes) return;
     const char* env = std::getenv("SGIPC_SPMV_GATHER");
     if (env && env[0] && env[0] != '0') return;  // keep the global-gather form (tests of both forms)
-    k_localize<<<g256(nl), 256, 0, s>>>(sell_cols.get(), slice_ptr.get(), perm.get(), halo_ptr.get(), halo_list.get(),
+    k_localize<<<g256(nl), 256, 0, s>>>(tile_rows, sell_cols.get(), slice_ptr.get(), perm.get(), halo_ptr.get(), halo_list.get(),
                                         n_slices);
     SGIPC_LAUNCH_CHECK();
     // heaviest tiles first inside each XCD's contiguous range of the launch order
     std::vector<int> ord((size_t)n_tiles);
+    const size_t per = (size_t)tile_rows / 64;  // slices of a tile
     const int q = n_tiles / 8, rem = n_tiles % 8;
     for (int xc = 0; xc < 8; ++xc) {
         const int b0 = xc * q + (xc < rem ? xc : rem), cnt = q + (xc < rem ? 1 : 0);
         for (int k = 0; k < cnt; ++k) ord[(size_t)b0 + k] = b0 + k;
         std::stable_sort(ord.begin() + b0, ord.begin() + b0 + cnt, [&](int u, int v) {
-            return sp[(size_t)(u + 1) * kSlices] - sp[(size_t)u * kSlices] >
-                   sp[(size_t)(v + 1) * kSlices] - sp[(size_t)v * kSlices];
+            return sp[(size_t)(u + 1) * per] - sp[(size_t)u * per] > sp[(size_t)(v + 1) * per] - sp[(size_t)v * per];
         });
     }
     order.reserve(n_tiles);
@@ -1197,21 +1187,21 @@ void FullMatrix::build_halo(hipStream_t s, int tbits)
 
 size_t FullMatrix::halo_dyn_bytes(size_t tv_size, int threads) const
 {
-    const size_t pieces = (size_t)(threads / 64 + kSlices - 1);
-    return (3 * (size_t)tl_max + pieces * 3 * 64 + 3 * ((size_t)kTile + (size_t)halo_max)) * tv_size;
+    const size_t pieces = (size_t)(threads / 64 + tile_rows / 64 - 1);
+    return (3 * (size_t)tl_max + pieces * 3 * 64 + 3 * ((size_t)tile_rows + (size_t)halo_max)) * tv_size;
 }
 
 size_t FullMatrix::halo_static_lds()
 {
     static size_t cached = 0;
     if (cached == 0) {
-        const void* fns[] = {reinterpret_cast<const void*>(&k_spmv_halo<double, double, false, false>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, true, false>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, false, true>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, true, true>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<float, double, true, false>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<float, double, true, true>),
-                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, false, false, true>)};
+        const void* fns[] = {reinterpret_cast<const void*>(&k_spmv_halo<double, double, kTileLarge, false, false>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, kTileLarge, true, false>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, kTileLarge, false, true>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, kTileLarge, true, true>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<float, double, kTileLarge, true, false>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<float, double, kTileLarge, true, true>),
+                             reinterpret_cast<const void*>(&k_spmv_halo<double, double, kTileLarge, false, false, true>)};
         size_t m = 0;
         for (const void* f : fns) {
             hipFuncAttributes fa;
@@ -1227,7 +1217,7 @@ int FullMatrix::partials() const { return n_tiles + n_long; }
 
 long FullMatrix::stored_blocks(hipStream_t s) const
 {
-    std::vector<int> h((size_t)n_tiles * kTile);
+    std::vector<int> h((size_t)n_tiles * tile_rows);
     SGIPC_HIP(hipMemcpyAsync(h.data(), plen.get(), sizeof(int) * h.size(), hipMemcpyDeviceToHost, s));
     SGIPC_HIP(hipStreamSynchronize(s));
     long t = 0;
@@ -1241,16 +1231,29 @@ int FullMatrix::launch(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, T
                        int n_rz, const Level1Sums* l1) const
 {
     SGIPC_CHECK(n_tiles > 0, SGIPC_EMPTY, "matrix was not built");
+    if (tile_rows == kTileLarge)
+        return launch_tiles<TM, TV, kTileLarge>(s, vals, a, x, b, y, dot_part, done, z, p_new, rzn, rzo, n_rz, l1);
+    if (tile_rows == kTileMid)
+        return launch_tiles<TM, TV, kTileMid>(s, vals, a, x, b, y, dot_part, done, z, p_new, rzn, rzo, n_rz, l1);
+    return launch_tiles<TM, TV, kTileSmall>(s, vals, a, x, b, y, dot_part, done, z, p_new, rzn, rzo, n_rz, l1);
+}
+
+template <typename TM, typename TV, int kTile>
+int FullMatrix::launch_tiles(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, TV* y, double* dot_part,
+                             const int* done, const TV* z, TV* p_new, const double* rzn, const double* rzo,
+                             int n_rz, const Level1Sums* l1) const
+{
     const int g = n_tiles;
     SGIPC_CHECK(l1 == nullptr || (use_halo && !dot_part && !p_new), SGIPC_BAD_ARG,
                 "level-1 sums ride on the plain halo-form SpMV only");
     const Level1Sums l1v = l1 ? *l1 : Level1Sums{};
     if (use_halo) {
-        constexpr int nt = HaloCfg<TM, TV>::NT;
-        const size_t dyn = halo_dyn_bytes(sizeof(typename HaloCfg<TM, TV>::TL), nt);
+        using Cfg = HaloCfg<TM, TV, kTile>;
+        constexpr int nt = Cfg::NT;
+        const size_t dyn = halo_dyn_bytes(sizeof(typename Cfg::TL), nt);
 #define SGIPC_HALO(DOT, FUSE, SUM1)                                                                                 \
     do {                                                                                                            \
-        const void* fn = reinterpret_cast<const void*>(&k_spmv_halo<TM, TV, DOT, FUSE, SUM1>);                      \
+        const void* fn = reinterpret_cast<const void*>(&k_spmv_halo<TM, TV, kTile, DOT, FUSE, SUM1>);               \
         static int max_dyn = -1;                                                                                    \
         if (max_dyn < 0) {                                                                                          \
             hipFuncAttributes fa;                                                                                   \
@@ -1260,7 +1263,7 @@ int FullMatrix::launch(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, T
             max_dyn = m;                                                                                            \
         }                                                                                                           \
         SGIPC_CHECK(dyn <= (size_t)max_dyn, SGIPC_CAPACITY, "halo SpMV needs more LDS than a CU has");              \
-        go(&k_spmv_halo<TM, TV, DOT, FUSE, SUM1>, g, nt, dyn, s, time_start, time_stop, vals,                      \
+        go(&k_spmv_halo<TM, TV, kTile, DOT, FUSE, SUM1>, g, nt, dyn, s, time_start, time_stop, vals,               \
            (const uint32_t*)sell_cols.get(), (const int*)slice_ptr.get(), (const int*)perm.get(),                   \
            (const int*)plen.get(), (const uint32_t*)tinfo.get(), (const int*)halo_ptr.get(),                        \
            (const int*)halo_list.get(), (const int*)order.get(), tl_max, a, x, b, y, dot_part, done, z, p_new, rzn, \
@@ -1281,7 +1284,7 @@ int FullMatrix::launch(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, T
         return dot_part ? g + n_long : 0;
     }
 #define SGIPC_TSYM(DOT, FUSE)                                                                                   \
-    go(&k_spmv_tsym<TM, TV, DOT, FUSE>, g, kThreads, 0, s, time_start, time_stop, vals,                            \
+    go(&k_spmv_tsym<TM, TV, kTile, DOT, FUSE>, g, kTile * kSplit, 0, s, time_start, time_stop, vals,               \
        (const uint32_t*)sell_cols.get(),                                                                            \
        (const int*)slice_ptr.get(), (const int*)slice_w.get(), (const int*)perm.get(), (const int*)plen.get(),       \
        (const uint32_t*)tinfo.get(), a, x, b, y, dot_part, done, z, p_new, rzn, rzo, n_rz, n_rows)

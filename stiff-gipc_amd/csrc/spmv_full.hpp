@@ -29,8 +29,8 @@ class FullMatrix {
     template <typename TV>
     int apply(hipStream_t s, TV a, const TV* x, TV b, TV* y, double* dot_part, const int* done) const;
     // y = a*A*x + b*y followed by the level-1 sums of y's rows (l1), in one
-    // launch of the halo form (the epilogue holds whole 512-row tiles, so
-    // whole level-0 domains).  Returns false, having launched nothing, when
+    // launch of the halo form (a tile is whole waves of rows, so whole
+    // level-0 domains).  Returns false, having launched nothing, when
     // the matrix is not in the halo form.
     template <typename TV>
     bool apply_level1_sums(hipStream_t s, TV a, const TV* x, TV b, TV* y, const int* done, const Level1Sums& l1) const;
@@ -58,6 +58,7 @@ class FullMatrix {
     int tl_max = 0;         // in-tile transposed slots the fullest tile uses
     long n_slots = 0;    // SELL slots (64 entries each, padding included)
     int n_slices = 0;
+    int tile_rows = 0;   // rows of a tile (chosen by the row count)
     int n_tiles = 0;
     bool has_f32 = false;
     // rows with too many blocks for the tiles: their full rows as CSR
@@ -92,6 +93,9 @@ class FullMatrix {
     int launch(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, TV* y, double* dot_part, const int* done,
                const TV* z, TV* p_new, const double* rzn, const double* rzo, int n_rz,
                const Level1Sums* l1 = nullptr) const;
+    template <typename TM, typename TV, int kTile>
+    int launch_tiles(hipStream_t s, const TM* vals, TV a, const TV* x, TV b, TV* y, double* dot_part, const int* done,
+                     const TV* z, TV* p_new, const double* rzn, const double* rzo, int n_rz, const Level1Sums* l1) const;
 
     DevBuf<uint64_t> keys_, skeys_, rkey_, rkey_sorted_;
     DevBuf<int> idx_, sidx_, cand_, cscan_, up_ptr_, col_ptr_, low_cnt_, len_, iota_, sorted_;
