@@ -472,9 +472,10 @@ typedef struct sgipc_pcg_opts {
     double ir_inner_tol; /* FP32_IR: floor of the inner tolerance (<= 0: none; each pass
                             asks for the residual reduction still missing)           */
     int fuse;          /* 1 (default): fold the x/r update into the first MAS kernel
-                          (MAS on every row, >= 3 levels); 2: also fold the p update
-                          into the SpMV; 0: separate vector kernels.  Same
-                          iterates either way. */
+                          (MAS on every row, >= 3 levels), and the p update into the
+                          SpMV where that is faster (matrices of few rows); 2: both
+                          always; 0: separate vector kernels.  Same iterates
+                          either way. */
     int flexible;      /* 1: flexible PCG, beta = -(z.Ap)/(p.Ap) (a preconditioner that
                           may change between iterations, e.g. the learned level); needs
                           the MAS on every row.  Same iterates as PCG for a fixed SPD

@@ -26,6 +26,7 @@ struct FullOp : SpmvOp<TV> {
         return m->apply<TV>(s, TV(1), p, TV(0), Ap, part, ctl ? &ctl->done : nullptr);
     }
     bool fuses_update_p() const override { return true; }
+    bool prefers_update_p() const override { return m->fused_update_pays(); }
     // r holds b on entry: r = b - A x with the FP64 values
     bool residual(hipStream_t s, const TV*, const TV* x, TV* r, const PcgCtl* ctl) const override
     {

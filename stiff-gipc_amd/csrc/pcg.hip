@@ -390,7 +390,7 @@ PcgResult PcgSolver<TV>::solve(hipStream_t s, const SpmvOp<TV>& A, Preconditione
     //   MAS:   x += alpha p_k, r -= alpha Ap, ||r||^2 in the restriction;
     //          stop rule in the first coarse restriction; z = M r, r.z
     // i.e. the p update of iteration k-1 is deferred into the SpMV of k.
-    const bool fuse_p = !flex && opt.fuse >= 2 && A.fuses_update_p();
+    const bool fuse_p = !flex && A.fuses_update_p() && (opt.fuse >= 2 || (opt.fuse == 1 && A.prefers_update_p()));
     bool fuse_xr = opt.fuse >= 1 && M != nullptr;  // cleared when the preconditioner declines
     const bool replace = sizeof(TV) == 8 && opt.true_op != nullptr && opt.replace_every > 0;
     bool p_pending = false;                   // p update of the previous iteration not yet applied

@@ -60,9 +60,8 @@ struct PcgOptions {
     int stop_mode = 1;     // 0 = reference |rz| <= tol*rz0, 1 = ||r|| <= tol*||b||
     int max_iter = 1000;
     int check_every = 8;
-    // 1: fold the x/r update into the preconditioner's first kernel;
-    // 2: also fold the p update into the SpMV (gathers z and p_old, which
-    // costs more than the separate update on this part); 0: neither
+    // 1: fold the x/r update into the preconditioner's first kernel, and the
+    // p update into the SpMV where that is faster; 2: both always; 0: neither
     int fuse = 1;
     // flexible PCG (preconditioner that may change between iterations):
     // beta = -(z_new . Ap) / (p . Ap) instead of rz_new / rz_old
@@ -130,6 +129,8 @@ struct SpmvOp {
     // into Ap = A p_new; returns the p.Ap partial count.  Called only when
     // fuses_update_p() is true.
     virtual bool fuses_update_p() const { return false; }
+    // the fused form is the faster one (taken with fuse = 1)
+    virtual bool prefers_update_p() const { return false; }
     virtual int apply_dot_update_p(hipStream_t, const TV*, const TV*, TV*, TV*, double*, const PcgCtl*,
                                    const double*, const double*, int) const
     {

@@ -267,9 +267,14 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
     __shared__ double dred[16];
     // slots per step (one for the fused p update, whose staging needs more registers)
     constexpr int kU = (sizeof(TM) == 4 && !kFuseP) ? 2 : 1;
+    double beta = 0.0, rz1 = 0.0, rz0 = 0.0;
+    if (kFuseP) {
+        for (int k = threadIdx.x; k < n_rz; k += kThreads) {
+            rz1 += rzn[k];
+            rz0 += rzo[k];
+        }
+    }
     if (done != nullptr && *done) return;
-    double beta = 0.0;
-    if (kFuseP) beta = block_sum_array(rzn, n_rz, dred) / block_sum_array(rzo, n_rz, dred);
     auto gx = [&](long k) -> TV {
         if (kFuseP) return (TV)((double)zf[k] + beta * (double)x[k]);
         return x[k];
@@ -320,11 +325,44 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
         issue(pos, sq, Wa, Ha, aa);
     }
     {
-        // stage the tile's own rows and its halo
+        // stage the tile's own rows and its halo; with the fused p update the
+        // first entries of a thread are in flight while beta is summed
         const long e3 = 3L * n_rows;
-        for (int t = threadIdx.x; t < 3 * kTile; t += kThreads) xl[t] = (TL)(b3 + t < e3 ? gx(b3 + t) : TV(0));
         const int h0 = halo_ptr[tile], hn = halo_ptr[tile + 1] - h0;
-        for (int k = threadIdx.x; k < hn; k += kThreads) {
+        if constexpr (kFuseP) {
+            constexpr int kOwn = (3 * kTile + kThreads - 1) / kThreads;
+            TV zo[kOwn], po[kOwn], zh[3], ph[3];
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                const int t = threadIdx.x + kThreads * q;
+                const bool in = t < 3 * kTile && b3 + t < e3;
+                zo[q] = in ? zf[b3 + t] : TV(0);
+                po[q] = in ? x[b3 + t] : TV(0);
+            }
+            const bool first = (int)threadIdx.x < hn;
+            const long j = first ? halo_list[h0 + threadIdx.x] : 0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                zh[c] = first ? zf[3 * j + c] : TV(0);
+                ph[c] = first ? x[3 * j + c] : TV(0);
+            }
+            rz1 = block_sum(rz1, dred);
+            rz0 = block_sum(rz0, dred);
+            beta = rz1 / rz0;
+#pragma unroll
+            for (int q = 0; q < kOwn; ++q) {
+                const int t = threadIdx.x + kThreads * q;
+                if (t < 3 * kTile) xl[t] = (TL)(TV)((double)zo[q] + beta * (double)po[q]);
+            }
+            if (first) {
+                TL* d = xl + 3 * (kTile + threadIdx.x);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) d[c] = (TL)(TV)((double)zh[c] + beta * (double)ph[c]);
+            }
+        } else {
+            for (int t = threadIdx.x; t < 3 * kTile; t += kThreads) xl[t] = (TL)(b3 + t < e3 ? gx(b3 + t) : TV(0));
+        }
+        for (int k = threadIdx.x + (kFuseP ? kThreads : 0); k < hn; k += kThreads) {
             const long j = halo_list[h0 + k];
             TL* d = xl + 3 * (kTile + k);
             d[0] = (TL)gx(3 * j);

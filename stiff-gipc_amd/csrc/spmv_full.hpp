@@ -45,6 +45,13 @@ class FullMatrix {
     int apply_update_p(hipStream_t s, bool f32_values, const TV* z, const TV* p_old, TV* p_new, TV* Ap,
                        double* dot_part, const int* done, const double* rz_new, const double* rz_old,
                        int n_rz) const;
+    // whether apply_update_p beats a separate p update: in the small row
+    // tiles, which leave the launch and the partial sums as the larger cost
+    // (16^3 grid, FP64: 6.8 us against 6.5 + 3.0; its solve 2.79 -> 2.62 ms).
+    // In 512-row tiles forming p twice at every halo vertex costs what the
+    // update did (262k rows, FP32 values: 32.9 us against 26.0 + 7.7, solve
+    // 27.9 -> 28.0 ms)
+    bool fused_update_pays() const { return use_halo && tile_rows < 512; }
     // partial count of apply() with dot_part
     int partials() const;
     // blocks stored in the layout (upper blocks + cross-tile transposed

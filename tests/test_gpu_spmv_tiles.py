@@ -54,3 +54,23 @@ def test_products(pkg, gpu_ctx, monkeypatch, form, n, long_row):
     assert M.layout()[0] == (1 if form == "halo" else 0)
     assert M.long_rows() == (1 if long_row and n // 3 > 128 else 0)
     M.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_mas", "fp32_ir"])
+@pytest.mark.parametrize("N,graph", [(9, True), (31, False)])
+def test_default_iteration_folds_the_p_update(pkg, N, precision, graph):
+    """On 64- and 128-row tiles the default iteration forms p inside the SpMV: the arithmetic of the separate update
+    except for the grouping of two sums, so the iterates after 25 steps differ by amplified rounding only (the bound
+    of the fused iteration's own test; 1e-6 where the tiles hold FP32 copies of p)."""
+    ls = pkg.LinearSystem(pkg.scenes.tet_grid_scene("fold", N, n_pairs=8), bank_size=16)
+    try:
+        kw = dict(precision=precision, graph=graph, ir_replace_every=0)
+        a = ls.solve(tol=1e-30, max_iter=26, fuse=1, **kw)
+        b = ls.solve(tol=1e-30, max_iter=26, fuse=0, **kw)
+        assert a.iterations == b.iterations
+        assert np.linalg.norm(a.x - b.x) <= (1e-13 if precision != "fp32_ir" else 1e-6) * np.linalg.norm(b.x)
+        a, b = (ls.solve(tol=1e-6, precision=precision, graph=graph, fuse=f) for f in (1, 0))
+        assert abs(a.iterations - b.iterations) <= 1
+        assert a.true_rel_residual <= 1e-6 and b.true_rel_residual <= 1e-6
+    finally:
+        ls.close()
