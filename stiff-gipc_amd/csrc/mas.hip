@@ -633,27 +633,13 @@ __global__ __launch_bounds__(256) void k_restrict0(PcgStopDesc sd, const int* __
         R[3 * (long)s + 2] = v2;
     }
     if (L > 1) {
-        // group-by level-1 node inside the wave (a node lives in one domain)
-        int node = real ? map1[s] : -1;
-        bool pending = node >= 0;
-        const int lane = threadIdx.x & 63;
-        while (true) {
-            const uint64_t act = __ballot(pending);
-            if (act == 0) break;
-            const int leader = __ffsll((unsigned long long)act) - 1;
-            const int key = __shfl(node, leader, 64);
-            const bool mine = pending && node == key;
-            TS s0 = wave_sum(mine ? v0 : TS(0));
-            TS s1 = wave_sum(mine ? v1 : TS(0));
-            TS s2 = wave_sum(mine ? v2 : TS(0));
-            if (lane == leader) {
-                const long o = 3 * (long)(npad + key);
-                R[o] = s0;
-                R[o + 1] = s1;
-                R[o + 2] = s2;
-            }
-            if (mine) pending = false;
-        }
+        // a level-1 node lies in one domain of B rows
+        group_key_sums<B>(real ? map1[s] : -1, v0, v1, v2, [&](int key, TS s0, TS s1, TS s2) {
+            const long o = 3 * (long)(npad + key);
+            R[o] = s0;
+            R[o + 1] = s1;
+            R[o + 2] = s2;
+        });
         // zero the padding slots of level 1
         const int c1 = meta[kMetaCnt + 1];
         const int pad = meta[kMetaOff + 2] - npad - c1;
@@ -724,12 +710,23 @@ __global__ __launch_bounds__(256) void k_restrict0_xr(FusedXR<TV> fx, const int*
         }
         return;
     }
-    const double rz = block_sum_array(fx.rz, fx.n_rz, smem);
-    const double pap = block_sum_array(fx.pap, fx.n_pap, smem);
-    const double alpha = rz / pap;
+    // the row's loads are in flight while alpha is summed
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int npad = meta[kMetaOff + 1];
     const bool real = s < n;
+    const long s3 = real ? 3 * (long)s : 0;
+    double r0[3], av[3], xv[3], pv[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        r0[c] = (double)fx.r[s3 + c];
+        av[c] = (double)fx.Ap[s3 + c];
+        xv[c] = (double)fx.x[s3 + c];
+        pv[c] = (double)fx.p[s3 + c];
+    }
+    const int node = real ? map1[s] : -1;
+    const double rz = block_sum_array(fx.rz, fx.n_rz, smem);
+    const double pap = block_sum_array(fx.pap, fx.n_pap, smem);
+    const double alpha = rz / pap;
     TS v0 = 0, v1 = 0, v2 = 0;
     double rrv = 0.0;
     if (real) {
@@ -737,8 +734,8 @@ __global__ __launch_bounds__(256) void k_restrict0_xr(FusedXR<TV> fx, const int*
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const long k = 3 * (long)s + c;
-            rv[c] = (double)fx.r[k] - alpha * (double)fx.Ap[k];
-            fx.x[k] = (TV)((double)fx.x[k] + alpha * (double)fx.p[k]);
+            rv[c] = r0[c] - alpha * av[c];
+            fx.x[k] = (TV)(xv[c] + alpha * pv[c]);
             fx.r[k] = (TV)rv[c];
             rrv += rv[c] * rv[c];
         }
@@ -752,26 +749,13 @@ __global__ __launch_bounds__(256) void k_restrict0_xr(FusedXR<TV> fx, const int*
         R[3 * (long)s + 2] = v2;
     }
     if (SUMS) {
-        int node = real ? map1[s] : -1;
-        bool pending = node >= 0;
-        const int lane = threadIdx.x & 63;
-        while (true) {
-            const uint64_t act = __ballot(pending);
-            if (act == 0) break;
-            const int leader = __ffsll((unsigned long long)act) - 1;
-            const int key = __shfl(node, leader, 64);
-            const bool mine = pending && node == key;
-            TS s0 = wave_sum(mine ? v0 : TS(0));
-            TS s1 = wave_sum(mine ? v1 : TS(0));
-            TS s2 = wave_sum(mine ? v2 : TS(0));
-            if (lane == leader) {
-                const long o = 3 * (long)(npad + key);
-                R[o] = s0;
-                R[o + 1] = s1;
-                R[o + 2] = s2;
-            }
-            if (mine) pending = false;
-        }
+        // a level-1 node lies in one domain of B rows
+        group_key_sums<B>(node, v0, v1, v2, [&](int key, TS s0, TS s1, TS s2) {
+            const long o = 3 * (long)(npad + key);
+            R[o] = s0;
+            R[o + 1] = s1;
+            R[o + 2] = s2;
+        });
         const int c1 = meta[kMetaCnt + 1];
         const int pad = meta[kMetaOff + 2] - npad - c1;
         if (s < pad) {
@@ -792,56 +776,29 @@ __global__ __launch_bounds__(256) void k_restrict0_xr(FusedXR<TV> fx, const int*
     }
 }
 
-// Level l-1 -> level l sums (l >= 2).
-template <typename TS>
-__global__ __launch_bounds__(256) void k_restrict_up(const int* __restrict__ done, const int* __restrict__ meta,
-                                                     int level, const int* __restrict__ going_next,
-                                                     TS* __restrict__ R, PcgStopDesc sd)
+// Level l-1 -> level l sums (l >= 2) for node a of level l-1 (a node's
+// children lie in one domain of B slots), and the padding slots of level l.
+// Whole waves call it.
+template <int B, typename TS>
+__device__ __forceinline__ void restrict_node(int a, int level, const int* __restrict__ meta,
+                                              const int* __restrict__ going_next, TS* __restrict__ R)
 {
-    if (sd.ctl != nullptr) {
-        // first coarse restriction after a fused x/r update: the stop rule
-        __shared__ double smem[16];
-        __shared__ int s_done;
-        if (threadIdx.x == 0) s_done = sd.ctl->done;
-        __syncthreads();
-        if (s_done) return;
-        const double rz = block_sum_array(sd.rz, sd.n_rz, smem);
-        const double rr = block_sum_array(sd.rr, sd.n_rr, smem);
-        if (pcg_stop_verdict(sd.ctl, rz, rr)) return;
-    } else if (done != nullptr && *done) {
-        return;
-    }
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
     const int cprev = meta[kMetaCnt + level - 1];
     const int offprev = meta[kMetaOff + level - 1];
-    const bool real = a < cprev;
     TS v0 = 0, v1 = 0, v2 = 0;
     int parent = -1;
-    if (real) {
+    if (a < cprev) {
         const long o = 3 * (long)(offprev + a);
         v0 = R[o];
         v1 = R[o + 1];
         v2 = R[o + 2];
         parent = going_next[offprev + a];
     }
-    bool pending = real;
-    const int lane = threadIdx.x & 63;
-    while (true) {
-        const uint64_t act = __ballot(pending);
-        if (act == 0) break;
-        const int leader = __ffsll((unsigned long long)act) - 1;
-        const int key = __shfl(parent, leader, 64);
-        const bool mine = pending && parent == key;
-        TS s0 = wave_sum(mine ? v0 : TS(0));
-        TS s1 = wave_sum(mine ? v1 : TS(0));
-        TS s2 = wave_sum(mine ? v2 : TS(0));
-        if (lane == leader) {
-            R[3 * (long)key] = s0;
-            R[3 * (long)key + 1] = s1;
-            R[3 * (long)key + 2] = s2;
-        }
-        if (mine) pending = false;
-    }
+    group_key_sums<B>(parent, v0, v1, v2, [&](int key, TS s0, TS s1, TS s2) {
+        R[3 * (long)key] = s0;
+        R[3 * (long)key + 1] = s1;
+        R[3 * (long)key + 2] = s2;
+    });
     const int c = meta[kMetaCnt + level];
     const int off = meta[kMetaOff + level];
     const int pad = meta[kMetaOff + level + 1] - off - c;
@@ -850,6 +807,47 @@ __global__ __launch_bounds__(256) void k_restrict_up(const int* __restrict__ don
         R[o] = 0;
         R[o + 1] = 0;
         R[o + 2] = 0;
+    }
+}
+
+// Whether the run has stopped: the flag, or after a fused x/r update (sd.ctl
+// set) the stop rule, evaluated by the first coarse restriction.
+__device__ __forceinline__ bool restrict_stops(const int* __restrict__ done, const PcgStopDesc& sd)
+{
+    if (sd.ctl == nullptr) return done != nullptr && *done;
+    __shared__ double smem[16];
+    __shared__ int s_done;
+    if (threadIdx.x == 0) s_done = sd.ctl->done;
+    __syncthreads();
+    if (s_done) return true;
+    const double rz = block_sum_array(sd.rz, sd.n_rz, smem);
+    const double rr = block_sum_array(sd.rr, sd.n_rr, smem);
+    return pcg_stop_verdict(sd.ctl, rz, rr);
+}
+
+template <int B, typename TS>
+__global__ __launch_bounds__(256) void k_restrict_up(const int* __restrict__ done, const int* __restrict__ meta,
+                                                     int level, const int* __restrict__ going_next,
+                                                     TS* __restrict__ R, PcgStopDesc sd)
+{
+    if (restrict_stops(done, sd)) return;
+    restrict_node<B>(blockIdx.x * blockDim.x + threadIdx.x, level, meta, going_next, R);
+}
+
+// Levels l0 .. L-1 in one workgroup, when level l0-1 has at most kTailNodes
+// nodes (one pass): the levels are all launch and latency (3.2 us each, 4.0 us
+// the two of a 16^3 grid in one launch; with the level-1 sums of all domains of
+// a wave at a time, its solve 2.66 -> 2.46 ms, one apply on 132k rows 60 -> 48 us).
+constexpr int kTailNodes = 1024;
+template <int B, typename TS>
+__global__ __launch_bounds__(1024) void k_restrict_tail(const int* __restrict__ done, const int* __restrict__ meta,
+                                                        int l0, int L, const int* __restrict__ going_next,
+                                                        TS* __restrict__ R, PcgStopDesc sd)
+{
+    if (restrict_stops(done, sd)) return;
+    for (int l = l0; l < L; ++l) {
+        restrict_node<B>(threadIdx.x, l, meta, going_next, R);
+        __syncthreads();
     }
 }
 
@@ -904,12 +902,9 @@ __device__ __forceinline__ void domain_product(const TS* __restrict__ sM, const 
             z2 += m[6] * r0 + m[7] * r1 + m[8] * r2;
         }
     }
-#pragma unroll
-    for (int off = G / 2; off >= 1; off >>= 1) {
-        z0 += __shfl_xor(z0, off, 64);
-        z1 += __shfl_xor(z1, off, 64);
-        z2 += __shfl_xor(z2, off, 64);
-    }
+    z0 = group_sum<G>(z0);
+    z1 = group_sum<G>(z1);
+    z2 = group_sum<G>(z2);
 }
 
 // FP16 storage of the level-0 inverse (coarse mode 2): C = D^-1 Minv D^-1
@@ -2164,6 +2159,33 @@ void Mas::set_bcoo(const double* vals, const int* rows, const int* cols, int nnz
     built = true;
 }
 
+// sd2: the stop rule, evaluated with the first restriction (level 2)
+template <int BB, typename TS>
+void Mas::restrict_level(hipStream_t s, int l, TS* R, const int* done, const PcgStopDesc& sd2)
+{
+    const int c = h_cnt[l - 1];
+    const int pad = h_off[l + 1] - h_off[l] - h_cnt[l];
+    const int work = c > pad ? c : pad;
+    k_restrict_up<BB, TS><<<grid_for(work > 0 ? work : 1, 256), 256, 0, s>>>(done, meta_.get(), l, going_next_.get(), R,
+                                                                        l == 2 ? sd2 : PcgStopDesc{});
+    SGIPC_LAUNCH_CHECK();
+}
+
+template <int BB, typename TS>
+void Mas::restrict_levels(hipStream_t s, TS* R, const int* done, const PcgStopDesc& sd2)
+{
+    int l = 2;
+    while (l < L && h_cnt[l - 1] > kTailNodes) restrict_level<BB, TS>(s, l++, R, done, sd2);
+    if (l == L - 1) {
+        restrict_level<BB, TS>(s, l, R, done, sd2);
+    } else if (l < L) {
+        // (padding slots: fewer than B per level)
+        k_restrict_tail<BB, TS><<<1, 1024, 0, s>>>(done, meta_.get(), l, L, going_next_.get(), R,
+                                                   l == 2 ? sd2 : PcgStopDesc{});
+        SGIPC_LAUNCH_CHECK();
+    }
+}
+
 template <int BB, typename TV, typename TS>
 int Mas::apply_t(hipStream_t s, const TV* r, TV* z, double* rz_part, const PcgStopDesc& sd)
 {
@@ -2251,23 +2273,15 @@ int Mas::finish_v_t(hipStream_t s, TS* R, TS* Z, const TS* minv, const int* done
     k_l1_residual<TS, false><<<g1w, 256, 0, s>>>(done, meta_.get(), c1, graph_.row_ptr.get(), graph_.col.get(),
                                                   graph_.blk.get(), graph_.s.get(), R, Z, G1, C2);
     SGIPC_LAUNCH_CHECK();
-    auto restrict_up_level = [&](int l) {
-        int c = h_cnt[l - 1];
-        int pad = h_off[l + 1] - h_off[l] - h_cnt[l];
-        int work = c > pad ? c : pad;
-        k_restrict_up<TS><<<grid_for(work > 0 ? work : 1, 256), 256, 0, s>>>(
-            done, meta_.get(), l, going_next_.get(), R, l == 2 ? sd2 : PcgStopDesc{});
-        SGIPC_LAUNCH_CHECK();
-    };
     int Lc = L;
     if (dense_m_ > 0) {
-        restrict_up_level(2);
+        restrict_level<BB, TS>(s, 2, R, done, sd2);
         k_dense_gemv<TS><<<dense_m_, 256, 0, s>>>(done, dense_m_, dense_ld_, dense_inv_.get(), R + 3L * h_off[2],
                                                                 Z + 3L * h_off[2]);
         SGIPC_LAUNCH_CHECK();
         Lc = 3;
     } else {
-        for (int l = 2; l < L; ++l) restrict_up_level(l);
+        restrict_levels<BB, TS>(s, R, done, sd2);
         if (ndom > ndom01) {
             k_local_solve<BB, TS><<<ndom - ndom01, 256, 0, s>>>(done, minv, R, Z, ndom01);
             SGIPC_LAUNCH_CHECK();
@@ -2334,17 +2348,7 @@ int Mas::finish_t(hipStream_t s, TS* R, TS* Z, const TS* minv, const int* done, 
     const int ndom01 = L > 1 ? h_off[2] / BB : ndom0;
     const int ndom = total / BB;
     const bool cyc = cycle_active();
-    auto restrict_up_level = [&](int l) {
-        int c = h_cnt[l - 1];
-        int pad = h_off[l + 1] - h_off[l] - h_cnt[l];
-        int work = c > pad ? c : pad;
-        k_restrict_up<TS><<<grid_for(work > 0 ? work : 1, 256), 256, 0, s>>>(
-            done, meta_.get(), l, going_next_.get(), R, l == 2 ? sd2 : PcgStopDesc{});
-        SGIPC_LAUNCH_CHECK();
-    };
-    auto restrict_up = [&]() {
-        for (int l = 2; l < L; ++l) restrict_up_level(l);
-    };
+    auto restrict_up = [&]() { restrict_levels<BB, TS>(s, R, done, sd2); };
     TS* G1 = nullptr;
     TS* C2 = nullptr;
     if (cyc) {
@@ -2367,7 +2371,7 @@ int Mas::finish_t(hipStream_t s, TS* R, TS* Z, const TS* minv, const int* done, 
         // (dense inverse) when it was built, else the additive levels >= 2
         int Lc = L;
         if (dense_m_ > 0) {
-            restrict_up_level(2);
+            restrict_level<BB, TS>(s, 2, R, done, sd2);
             k_dense_gemv<TS><<<dense_m_, 256, 0, s>>>(done, dense_m_, dense_ld_, dense_inv_.get(),
                                                                     R + 3L * h_off[2], Z + 3L * h_off[2]);
             SGIPC_LAUNCH_CHECK();

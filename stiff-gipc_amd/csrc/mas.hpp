@@ -116,6 +116,10 @@ class Mas {
     int finish_t(hipStream_t s, TS* R, TS* Z, const TS* minv, const int* done, const PcgStopDesc& sd2, const TV* r,
                  TV* z, double* rz_part);
     // coarse mode 2 from the level-0 slots of r on
+    template <int BB, typename TS>
+    void restrict_level(hipStream_t s, int l, TS* R, const int* done, const PcgStopDesc& sd2);
+    template <int BB, typename TS>
+    void restrict_levels(hipStream_t s, TS* R, const int* done, const PcgStopDesc& sd2);
     template <int BB, typename TV, typename TS>
     int finish_v_t(hipStream_t s, TS* R, TS* Z, const TS* minv, const int* done, const PcgStopDesc& sd2,
                    const TV* r, TV* z, double* rz_part);

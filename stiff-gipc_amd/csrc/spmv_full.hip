@@ -507,8 +507,8 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
     if constexpr (kSum1) {
         // the tile's new rows back in row order (piece is free once every
         // row has been summed), then the level-1 sums: a level-1 node lies in
-        // one 32-row level-0 domain, so in one wave of 64 rows, whose lanes
-        // group by node (the leader writes the node's sum)
+        // one level-0 domain of 16 or 32 rows, so in one aligned group of 32
+        // lanes
         __syncthreads();
         TL* const yb = piece;
         if (ylr >= 0) {
@@ -523,26 +523,12 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
             const TV v0 = real ? (TV)yb[3 * threadIdx.x] : TV(0);
             const TV v1 = real ? (TV)yb[3 * threadIdx.x + 1] : TV(0);
             const TV v2 = real ? (TV)yb[3 * threadIdx.x + 2] : TV(0);
-            int node = real ? l1.map1[u] : -1;
-            bool pending = node >= 0;
-            const int lane = threadIdx.x & 63;
-            while (true) {
-                const uint64_t act = __ballot(pending);
-                if (act == 0) break;
-                const int leader = __ffsll((unsigned long long)act) - 1;
-                const int key = __shfl(node, leader, 64);
-                const bool mine = pending && node == key;
-                const TV s0 = wave_sum(mine ? v0 : TV(0));
-                const TV s1 = wave_sum(mine ? v1 : TV(0));
-                const TV s2 = wave_sum(mine ? v2 : TV(0));
-                if (lane == leader) {
-                    const long o = 3 * (long)(l1.npad + key);
-                    y[o] = s0;
-                    y[o + 1] = s1;
-                    y[o + 2] = s2;
-                }
-                if (mine) pending = false;
-            }
+            group_key_sums<32>(real ? l1.map1[u] : -1, v0, v1, v2, [&](int key, TV s0, TV s1, TV s2) {
+                const long o = 3 * (long)(l1.npad + key);
+                y[o] = s0;
+                y[o + 1] = s1;
+                y[o + 2] = s2;
+            });
         }
         if (tile == 0) {
             for (int k = threadIdx.x; k < l1.pad; k += kThreads) {

@@ -81,6 +81,52 @@ __device__ __forceinline__ T wave_max(T v)
     return wave_reduce(v, [](T x, T y) { return y > x ? y : x; });
 }
 
+// Sum over the aligned group of W lanes, in all of them (every lane of the
+// group active), in the order of the __shfl_xor steps from W / 2 down to 1.
+template <int W, typename T>
+__device__ __forceinline__ T group_sum(T v)
+{
+    static_assert(W == 8 || W == 16 || W == 32, "half a row, a row, a row pair");
+    if constexpr (W == 8) {
+        v += dpp_row<0x1B>(dpp_row<0x141>(v));  // row_half_mirror, quad_perm [3,2,1,0]: lane ^ 4
+        v += dpp_row<0x4E>(v);                  // quad_perm: lane ^ 2
+        return v + dpp_row<0xB1>(v);
+    } else {
+        if constexpr (W == 32) {
+            T a, b;
+            swap_halves<16>(v, a, b);
+            v = a + b;
+        }
+        v += dpp_row<0x128>(v);  // row_ror:8
+        v += dpp_row<0x124>(v);
+        v += dpp_row<0x122>(v);
+        return v + dpp_row<0x121>(v);
+    }
+}
+
+// Sums of three values by key within aligned groups of W lanes, all groups of
+// the wave at a time: write(key, s0, s1, s2) runs once per distinct key >= 0
+// of a group, as many rounds as the group with the most keys has.
+template <int W, typename T, typename F>
+__device__ __forceinline__ void group_key_sums(int key, T v0, T v1, T v2, F write)
+{
+    const int lane = threadIdx.x & 63, base = lane & ~(W - 1);
+    bool pending = key >= 0;
+    while (true) {
+        const uint64_t act = __ballot(pending);
+        if (act == 0) break;
+        const uint32_t mask = (uint32_t)(act >> base) & (uint32_t)((1ull << W) - 1);
+        const int leader = mask != 0 ? base + __ffs(mask) - 1 : lane;
+        const int k = __shfl(key, leader, 64);
+        const bool mine = pending && key == k;
+        const T s0 = group_sum<W>(mine ? v0 : T(0));
+        const T s1 = group_sum<W>(mine ? v1 : T(0));
+        const T s2 = group_sum<W>(mine ? v2 : T(0));
+        if (mine && lane == leader) write(k, s0, s1, s2);
+        if (mine) pending = false;
+    }
+}
+
 // Workgroup b of n -> its place in a contiguous run per XCD: the 8 XCDs take
 // workgroups in turn, so XCD b % 8 gets run [x n / 8 ..) and its L2 holds what
 // neighbours share.  A bijection on [0, n).
