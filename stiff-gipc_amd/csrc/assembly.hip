@@ -50,11 +50,9 @@ __device__ __forceinline__ void jacobi3(double A[3][3], double V[3][3])
             const int q = pq == 0 ? 1 : 2;
             const double apq = A[p][q];
             if (apq == 0.0) continue;
-            // tan of the rotation angle, sign(d) 2 a_pq / (|d| + sqrt(d^2 + 4 a_pq^2)): one
-            // division and two roots instead of three divisions and two roots
-            const double d = A[q][q] - A[p][p], a2 = 2.0 * apq, h = fabs(d) + sqrt(d * d + a2 * a2);
-            const double t = h > 0.0 ? (d >= 0.0 ? a2 : -a2) / h : 1.0;
-            const double c = rsqrt(t * t + 1.0), s = t * c;
+            const double theta = (A[q][q] - A[p][p]) / (2.0 * apq);
+            const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
+            const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 const double akp = A[k][p], akq = A[k][q];
@@ -126,7 +124,7 @@ __device__ void svd3_rv(const double F[3][3], double U[3][3], double S[3], doubl
     double n0 = sqrt(u0[0] * u0[0] + u0[1] * u0[1] + u0[2] * u0[2]);
     if (n0 > 1e-300) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) u0[k] *= 1.0 / n0;
+        for (int k = 0; k < 3; ++k) u0[k] /= n0;
     } else {
         u0[0] = 1.0; u0[1] = 0.0; u0[2] = 0.0;
     }
@@ -137,7 +135,7 @@ __device__ void svd3_rv(const double F[3][3], double U[3][3], double S[3], doubl
     double n1 = sqrt(u1[0] * u1[0] + u1[1] * u1[1] + u1[2] * u1[2]);
     if (n1 > 1e-14 * (n0 > 0 ? n0 : 1.0)) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) u1[k] *= 1.0 / n1;
+        for (int k = 0; k < 3; ++k) u1[k] /= n1;
     } else {
         // any unit vector orthogonal to u0
         double e[3] = {fabs(u0[0]) < 0.9 ? 1.0 : 0.0, fabs(u0[0]) < 0.9 ? 0.0 : 1.0, 0.0};
@@ -159,24 +157,31 @@ __device__ void svd3_rv(const double F[3][3], double U[3][3], double S[3], doubl
     S[2] = u2[0] * fv[0][2] + u2[1] * fv[1][2] + u2[2] * fv[2][2];
 }
 
+__device__ __forceinline__ int up12(int r, int c) { return r * 12 - r * (r - 1) / 2 + (c - r); }
+
+// acc += lam * g g^T (upper triangle of 12x12)
+__device__ __forceinline__ void rank1_upper(double acc[78], const double g[12], double lam)
+{
+#pragma unroll
+    for (int r = 0; r < 12; ++r) {
+        const double lr = lam * g[r];
+#pragma unroll
+        for (int c = r; c < 12; ++c) acc[up12(r, c)] += lr * g[c];
+    }
+}
+
 // ------------------------------------------------------------------ tet kernel
-// One thread per tet.  In the singular bases (F = U S V^T) the projected
-// 9x9 Hessian couples u_i v_i with u_j v_j (the scaling modes, a 3x3 matrix
-// A+) and u_i v_j with u_j v_i (twist and flip of one axis) and nothing else,
-// so with w_a = V^T d_a each vertex block is U M_ab U^T with
-//   M_ab[i][i] = A+_ii w_a[i] w_b[i] + sum_{j != i} p_ij w_a[j] w_b[j]
-//   M_ab[i][j] = A+_ij w_a[i] w_b[j] + m_ij w_a[j] w_b[i]
-// (p, m: half the sum and difference of the flip and twist eigenvalues): a
-// block is formed when it is stored, from 33 numbers.  The kernel is bound by
-// its stores: the 10 blocks of a tet are 720 consecutive bytes, and a thread
-// writing them for itself touches 64 lines with every instruction.  A wave
-// instead passes two blocks of its 64 tets at a time through LDS and stores
-// 144-byte runs; the gradient is summed per workgroup (VertexSums) before it
-// goes to memory.  1.5 M tets, 1.37 GB: 0.41 ms with the gradient, 0.39
-// without (0.90 and 0.60 ms with a 12x12 sum of rank-one modes in registers,
-// stores per thread and an atomic to memory per gradient component); 0.27 ms
-// of it remain without the block stores.  Whole 720-byte runs (46 KB of LDS
-// for one wave) took the same time: fewer waves fit.
+// One thread per tet; the 12x12 Hessian is summed from the clamped rank-one
+// modes in registers.  Bound by its scattered writes: the 10 blocks of a tet
+// are 720 consecutive bytes, and a thread writing them for itself touches 64
+// lines with every instruction, so a wave passes two blocks of its 64 tets at
+// a time through LDS and stores 144-byte runs; and an atomic to memory per
+// gradient component costs more than all stores, so a thread parks its twelve
+// in LDS and the workgroup sums them by vertex (VertexSums) after the blocks.
+// 1.5 M tets with gradient, 1.37 GB: 0.90 -> 0.64 ms; the staged stores
+// alone change nothing (0.90).  The modes keep the order of their sums:
+// forming the blocks in the singular bases (U M_ab U^T) took 0.41 ms but
+// raised the error against 64 bits from 1.2e-15 to 1.4e-15.
 constexpr int kTetThreads = 128;
 __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const double* __restrict__ x,
                                                  const uint4* __restrict__ tets, const double* __restrict__ dm_inv,
@@ -186,6 +191,7 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
                                                  int* __restrict__ trows, int* __restrict__ tcols)
 {
     __shared__ double stage[kTetThreads / 64][64 * 18];
+    __shared__ double forces[kTetThreads][13];
     __shared__ VertexSums<256> sums;
     if (grad) sums.init();
     const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
@@ -239,18 +245,14 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
         cof[2][1] = F[0][2] * F[1][0] - F[0][0] * F[1][2];
         cof[2][2] = F[0][0] * F[1][1] - F[0][1] * F[1][0];
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            double f[3];
+        for (int a = 0; a < 4; ++a)
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 double s = 0.0;
 #pragma unroll
                 for (int j = 0; j < 3; ++j) s += (mu * F[d][j] + c * cof[d][j]) * D[a][j];
-                f[d] = scale * s;
+                if (act) forces[threadIdx.x][3 * a + d] = scale * s;
             }
-            if (act) sums.add((int)vid[a], f[0], f[1], f[2], grad);
-        }
-        sums.flush(grad);
     }
 
     double U[3][3], S[3], V[3][3];
@@ -262,18 +264,31 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
 #pragma unroll
         for (int i = 0; i < 3; ++i) w[a][i] = V[0][i] * D[a][0] + V[1][i] * D[a][1] + V[2][i] * D[a][2];
 
+    double acc[78];
+#pragma unroll
+    for (int e = 0; e < 78; ++e) acc[e] = 0.0;
+    const double rs2 = 0.70710678118654752440;
     // twist (Q = (u_j v_i^T - u_i v_j^T)/sqrt2) and flip (Q = (u_i v_j^T + u_j v_i^T)/sqrt2)
     // modes for axis k with (i, j) the other two axes; eigenvalues mu +/- c S[k]
-    auto clamp = [](double l) { return l <= 0.0 ? 0.0 : l; };  // keeps a NaN
-    double p[3], m[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const double lt = clamp(mu + c * S[k]), lf = clamp(mu - c * S[k]);
-        p[k] = 0.5 * (lf + lt) * scale;
-        m[k] = 0.5 * (lf - lt) * scale;
+        const int i = k == 0 ? 1 : 0;
+        const int j = k == 2 ? 1 : 2;
+#pragma unroll
+        for (int flip = 0; flip < 2; ++flip) {
+            const double l = flip ? (mu - c * S[k]) : (mu + c * S[k]);
+            if (l <= 0.0) continue;
+            double g[12];
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    g[3 * a + d] = flip ? rs2 * (U[d][i] * w[a][j] + U[d][j] * w[a][i])
+                                        : rs2 * (U[d][j] * w[a][i] - U[d][i] * w[a][j]);
+            rank1_upper(acc, g, l);
+        }
     }
     // scaling modes: eigen-decomposition of the 3x3 block in singular space
-    double Ap[3][3];
     {
         const double ev = lam * (2.0 * J - 1.0) - mu;
         double A[3][3];
@@ -286,44 +301,18 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
         double E[3][3];
         jacobi3(A, E);
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+        for (int m = 0; m < 3; ++m) {
+            const double l = A[m][m];
+            if (l <= 0.0) continue;
+            double g[12];
 #pragma unroll
-            for (int j = i; j < 3; ++j) {
-                double v = 0.0;
+            for (int a = 0; a < 4; ++a)
 #pragma unroll
-                for (int q = 0; q < 3; ++q) v += clamp(A[q][q]) * E[i][q] * E[j][q];
-                Ap[i][j] = Ap[j][i] = v * scale;
-            }
+                for (int d = 0; d < 3; ++d)
+                    g[3 * a + d] = E[0][m] * U[d][0] * w[a][0] + E[1][m] * U[d][1] * w[a][1] + E[2][m] * U[d][2] * w[a][2];
+            rank1_upper(acc, g, l);
+        }
     }
-    // block (a, b), row r and column c: U M_ab U^T
-    auto block = [&](int a, int b, double H[3][3]) {
-        double M[3][3], T[3][3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                if (i == j) {
-                    const int u = (i + 1) % 3, v = (i + 2) % 3;  // p of (i, u) belongs to axis v
-                    M[i][i] = Ap[i][i] * w[a][i] * w[b][i] + p[v] * w[a][u] * w[b][u] + p[u] * w[a][v] * w[b][v];
-                } else {
-                    M[i][j] = Ap[i][j] * w[a][i] * w[b][j] + m[3 - i - j] * w[a][j] * w[b][i];
-                }
-            }
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) T[r][j] = U[r][0] * M[0][j] + U[r][1] * M[1][j] + U[r][2] * M[2][j];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                if (a == b && q < r) {
-                    H[r][q] = H[q][r];  // diagonal blocks exactly symmetric
-                    continue;
-                }
-                H[r][q] = T[r][0] * U[q][0] + T[r][1] * U[q][1] + T[r][2] * U[q][2];
-            }
-    };
     // 10 upper blocks, local (ii <= jj), stored at (min, max) of the global
     // ids: transposed when the ids are in the other order
     const int lane = threadIdx.x & 63;
@@ -344,13 +333,14 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
         for (int k = 0; k < 2; ++k) {
             const int ii = kI[k0 + k], jj = kJ[k0 + k];
             const bool keep = vid[ii] <= vid[jj];
-            double H[3][3];
-            block(ii, jj, H);
             double* const q = st + 18 * lane + 9 * k;
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
-                for (int cc = 0; cc < 3; ++cc) q[keep ? cc * 3 + r : r * 3 + cc] = H[r][cc];
+                for (int cc = 0; cc < 3; ++cc) {
+                    const int R = 3 * ii + r, C = 3 * jj + cc;
+                    q[keep ? cc * 3 + r : r * 3 + cc] = scale * acc[R <= C ? up12(R, C) : up12(C, R)];
+                }
         }
         wave_lds_sync();
         double* const dst = tvals + 90 * w0 + 9 * k0;
@@ -371,6 +361,15 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
         int* const dst = (side == 0 ? trows : tcols) + 10 * w0;
         for (int e = lane; e < 10 * nw; e += 64) dst[e] = si[e];
         wave_lds_sync();
+    }
+    if (grad) {
+        if (act)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const double* const f = forces[threadIdx.x] + 3 * a;
+                sums.add((int)vid[a], f[0], f[1], f[2], grad);
+            }
+        sums.flush(grad);
     }
 }
 
