@@ -417,8 +417,8 @@ __device__ __forceinline__ double read_lane(double v, int lane)
 // definite) sets *nonpos.  A step is 36 FMAs per thread, so what stands beside
 // them counts: only the wave that owns the pivot row divides (a division in
 // every wave took as long as the FMAs), and the six steps of a tile are
-// unrolled, so no step selects its row and column of a at run time.  4 000 /
-// 8 200 domains of 32 vertices: 537 / 1190 -> 326 / 707 us, one 96 x 96 pivot
+// unrolled, so no step selects its row and column of a at run time.  3 456 /
+// 8 192 domains of 32 vertices: 537 / 1190 -> 326 / 707 us, one 96 x 96 pivot
 // block 87 -> 42 us, the same bits; gathering and storing the blocks is 80 of
 // the 326.  Four waves per SIMD instead of three spill (1126 us).
 template <int B>
