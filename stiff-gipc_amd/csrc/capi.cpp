@@ -517,9 +517,11 @@ int pcg_solve_impl(Context& c, SolveWorkspace& ws, const double* vals, const int
     // MAS covers every row; an FP32 MAS apply reads its FP32 copy
     const bool mas_fine = prec.mas != nullptr && prec.mas->coarse_mode == 2 && prec.mas_row_offset == 0 &&
                           !(prec.abd != nullptr && prec.abd->n_bodies > 0) && prec.mas->n == n_rows;
-    const bool want_f32 = o.precision == SGIPC_FP32_IR || (mas_fine && prec.mas->precision != SGIPC_FP64);
-    if (!(ws.prebuilt && ws.full.n_rows == n_rows && ws.full.nnz == nnz && (ws.full.has_f32 || !want_f32)))
-        ws.full.build(s, vals, rows, cols, nnz, n_rows, want_f32);
+    const bool f32_cycle = mas_fine && prec.mas->precision != SGIPC_FP64;
+    const bool want_f32 = o.precision == SGIPC_FP32_IR || f32_cycle;
+    if (!(ws.prebuilt && ws.full.n_rows == n_rows && ws.full.nnz == nnz && (ws.full.has_f32 || !want_f32) &&
+          (ws.full.has_fixed_tiles() || !f32_cycle)))
+        ws.full.build(s, vals, rows, cols, nnz, n_rows, want_f32, f32_cycle);
     if (prec.mas != nullptr && (mas_fine || !prec.mas->build_own_fine)) prec.mas->fine_ = mas_fine ? &ws.full : nullptr;
     if (o.precision != SGIPC_FP32_IR) {
         FullOp<double> A;

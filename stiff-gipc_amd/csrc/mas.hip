@@ -2153,7 +2153,8 @@ void Mas::set_bcoo(const double* vals, const int* rows, const int* cols, int nnz
     if (want_ap && build_own_fine && sub_nnz_ > 0) {
         const int* fr = offset > 0 ? sub_rows_.get() : rows;
         const int* fc = offset > 0 ? sub_cols_.get() : cols;
-        own_fine_.build(ctx->stream, vals + 9 * sub_e0_, fr, fc, sub_nnz_, n, precision != SGIPC_FP64);
+        const bool f32 = precision != SGIPC_FP64;
+        own_fine_.build(ctx->stream, vals + 9 * sub_e0_, fr, fc, sub_nnz_, n, f32, f32);
         fine_ = &own_fine_;
     }
     finish_dense_level2(ctx->stream);

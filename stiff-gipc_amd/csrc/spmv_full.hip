@@ -989,7 +989,7 @@ void go(void (*kernel)(KArgs...), int grid, int block, size_t shmem, hipStream_t
 }  // namespace
 
 void FullMatrix::build(hipStream_t s, const double* vals, const int* rows, const int* cols, int nnz_up, int n,
-                       bool want_f32)
+                       bool want_f32, bool fixed_tiles)
 {
     SGIPC_CHECK(nnz_up > 0 && n > 0, SGIPC_EMPTY, "empty matrix");
     n_rows = n;
@@ -997,7 +997,9 @@ void FullMatrix::build(hipStream_t s, const double* vals, const int* rows, const
     has_f32 = want_f32;
     int kbits = 1;
     while (kbits < 31 && (1L << kbits) < (long)n) ++kbits;
-    tile_rows = n <= kTileLarge ? kTileLarge : n < kRowsSmall ? kTileSmall : (n < kRowsMid ? kTileMid : kTileLarge);
+    tile_rows = fixed_tiles || n <= kTileLarge ? kTileLarge
+                : n < kRowsSmall               ? kTileSmall
+                                               : (n < kRowsMid ? kTileMid : kTileLarge);
     n_tiles = (n + tile_rows - 1) / tile_rows;
     const int n_pos = n_tiles * tile_rows;
     n_slices = n_pos / 64;

@@ -20,9 +20,12 @@ struct Level1Sums {
 class FullMatrix {
   public:
     // Lay out a unique upper BCOO (rows sorted, row <= col, indices < n).
-    // want_f32 also keeps FP32 values.
+    // want_f32 also keeps FP32 values.  fixed_tiles: 512-row tiles at every
+    // row count, for products with FP32 vectors whose rounding is amplified
+    // (the two-grid cycle): a row's FP32 sum is then cut the same way whatever
+    // the size of the matrix.
     void build(hipStream_t s, const double* vals, const int* rows, const int* cols, int nnz_up, int n,
-               bool want_f32);
+               bool want_f32, bool fixed_tiles = false);
     // y = a*A*x + b*y; dot_part (optional) receives one x^T(A x) partial per
     // tile; returns the partial count (0 without dot_part).  Returns at once
     // when *done != 0.
@@ -52,6 +55,8 @@ class FullMatrix {
     // update did (262k rows, FP32 values: 32.9 us against 26.0 + 7.7, solve
     // 27.9 -> 28.0 ms)
     bool fused_update_pays() const { return use_halo && tile_rows < 512; }
+    // whether the layout is the one that build() with fixed_tiles makes
+    bool has_fixed_tiles() const { return tile_rows == 512; }
     // partial count of apply() with dot_part
     int partials() const;
     // blocks stored in the layout (upper blocks + cross-tile transposed
@@ -65,7 +70,7 @@ class FullMatrix {
     int tl_max = 0;         // in-tile transposed slots the fullest tile uses
     long n_slots = 0;    // SELL slots (64 entries each, padding included)
     int n_slices = 0;
-    int tile_rows = 0;   // rows of a tile (chosen by the row count)
+    int tile_rows = 0;   // rows of a tile (chosen by the row count, or 512)
     int n_tiles = 0;
     bool has_f32 = false;
     // rows with too many blocks for the tiles: their full rows as CSR

@@ -806,8 +806,10 @@ int system_solve(sgipc_system* sys, const double* b, double* x, double* grad, co
         std::thread layout([&] {
             try {
                 sys->ctx->c.activate();
+                // an FP32 two-grid cycle over all rows multiplies by this matrix too
                 ws.full.build(ws.layout_side.s, sys->bvals.get(), sys->brows.get(), sys->bcols.get(), sys->nnz,
-                              sys->n_sys, o.precision != SGIPC_FP64);
+                              sys->n_sys, o.precision != SGIPC_FP64,
+                              mprec != SGIPC_FP64 && sys->mas->m->coarse_mode == 2 && off0 == 0);
             } catch (...) {
                 layout_err = std::current_exception();
             }
