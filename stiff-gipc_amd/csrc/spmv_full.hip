@@ -222,18 +222,20 @@ __global__ __launch_bounds__(kTile * kSplit) void k_spmv_tsym(const TM* __restri
 // wave order.  Each step's loads are issued before the previous step is used.
 // Tiles run in `order` (heaviest first inside each XCD's range), so the
 // lightest tiles fill the second round of workgroups.
-// Dynamic LDS: tl[3 tcap], piece[3 * 64 kPieces], xl[3 (kTile + hcap)] of TV.
+// Dynamic LDS: tl[3 tcap], piece[3 * 64 kPieces], xl[3 (kTile + hcap)] of TL.
 // Launch shape and LDS element type of the halo kernel per (matrix, vector)
-// type: the FP64 kernel keeps exact FP64 copies in LDS (one 1024-thread
-// workgroup per CU); the kernels with FP32 values keep FP32 copies (the
-// vector and the in-tile transposed products rounded to FP32, accumulation
-// in the vector type) in 512-thread workgroups, two of which fit a CU's LDS
-// and registers, so one workgroup's staging and reduction overlap the other's
-// stream.
+// type and tile: the FP64 kernel keeps exact FP64 copies in LDS (one
+// 1024-thread workgroup per CU); with FP32 values 512-row tiles keep FP32
+// copies (the vector, the partial row sums and the in-tile transposed products
+// rounded to FP32, accumulation in the vector type) in 512-thread workgroups,
+// two of which fit a CU's LDS and registers, so one workgroup's staging and
+// reduction overlap the other's stream.  Small tiles keep the vector type: a
+// slice is shared by up to eight waves there, each of whose pieces would be
+// rounded, and their LDS has room (same times).
 template <typename TM, typename TV, int kTile>
 struct HaloCfg {
     static constexpr int NT = kTile == kTileLarge && sizeof(TM) == 8 ? 1024 : 512;
-    using TL = typename std::conditional<sizeof(TM) == 4, float, TV>::type;
+    using TL = typename std::conditional<sizeof(TM) == 4 && kTile == kTileLarge, float, TV>::type;
 };
 
 template <typename TM, typename TV, int kTile, bool kDot, bool kFuseP, bool kSum1 = false>
@@ -267,6 +269,14 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
     __shared__ double dred[16];
     // slots per step (one for the fused p update, whose staging needs more registers)
     constexpr int kU = (sizeof(TM) == 4 && !kFuseP) ? 2 : 1;
+    // FP32 values with FP64 sums: multiply-adds written out, since the compiler
+    // contracts the two step widths differently and the iteration with the
+    // fused p update would round unlike the one without
+    constexpr bool kFma = sizeof(TM) == 4 && sizeof(TL) == 8;
+    auto dot3 = [](TV p, TV a1, TV q, TV a2, TV r, TV a3) -> TV {
+        if constexpr (kFma) return fma(r, a3, fma(q, a2, p * a1));
+        else return p * a1 + q * a2 + r * a3;
+    };
     double beta = 0.0, rz1 = 0.0, rz0 = 0.0;
     if (kFuseP) {
         for (int k = threadIdx.x; k < n_rz; k += kThreads) {
@@ -405,14 +415,14 @@ __global__ __launch_bounds__((HaloCfg<TM, TV, kTile>::NT), 4) void k_spmv_halo(c
                 const int lc = 3 * ((w >> 16) & 0x3FFF);
                 const TV x0 = m * (TV)xl[lc], x1 = m * (TV)xl[lc + 1], x2 = m * (TV)xl[lc + 2];
                 const TM* h = Ha[u];
-                a0 += (TV)h[0] * x0 + (TV)h[3] * x1 + (TV)h[6] * x2;
-                a1 += (TV)h[1] * x0 + (TV)h[4] * x1 + (TV)h[7] * x2;
-                a2 += (TV)h[2] * x0 + (TV)h[5] * x1 + (TV)h[8] * x2;
+                a0 += dot3((TV)h[0], x0, (TV)h[3], x1, (TV)h[6], x2);
+                a1 += dot3((TV)h[1], x0, (TV)h[4], x1, (TV)h[7], x2);
+                a2 += dot3((TV)h[2], x0, (TV)h[5], x1, (TV)h[8], x2);
                 if (aa[u] && (w & kInTile)) {
                     const int ts = w & 0xFFFF;
-                    tl[3 * ts] = (TL)((TV)h[0] * xi0 + (TV)h[1] * xi1 + (TV)h[2] * xi2);
-                    tl[3 * ts + 1] = (TL)((TV)h[3] * xi0 + (TV)h[4] * xi1 + (TV)h[5] * xi2);
-                    tl[3 * ts + 2] = (TL)((TV)h[6] * xi0 + (TV)h[7] * xi1 + (TV)h[8] * xi2);
+                    tl[3 * ts] = (TL)dot3((TV)h[0], xi0, (TV)h[1], xi1, (TV)h[2], xi2);
+                    tl[3 * ts + 1] = (TL)dot3((TV)h[3], xi0, (TV)h[4], xi1, (TV)h[5], xi2);
+                    tl[3 * ts + 2] = (TL)dot3((TV)h[6], xi0, (TV)h[7], xi1, (TV)h[8], xi2);
                 }
             }
             if (!more) break;

@@ -56,6 +56,33 @@ def test_products(pkg, gpu_ctx, monkeypatch, form, n, long_row):
     M.close()
 
 
+@pytest.mark.parametrize("form", ["halo", "gather"])
+@pytest.mark.parametrize("n,long_row", [(513, False), (1000, True), (27999, False), (28127, False), (60001, True)])
+def test_small_tiles_sum_in_fp64(pkg, gpu_ctx, monkeypatch, form, n, long_row):
+    """FP32 values against an FP64 vector, both exact in FP32: with the 64- and 128-row tiles' FP64 partial sums no
+    rounding to FP32 is left, only a few hundred of 2^-53 of each row's absolute sum."""
+    monkeypatch.setenv("SGIPC_SPMV_GATHER", "1" if form == "gather" else "0")
+    rng = np.random.default_rng(n)
+    v, r, c, _ = matrix(n, rng, long_row)
+    f = v.astype(np.float32).astype(np.float64)
+    x = rng.standard_normal(3 * n).astype(np.float32).astype(np.float64)
+    H, d = f.reshape(-1, 3, 3).transpose(0, 2, 1), r == c
+    k = np.arange(3)
+    i, j = (np.broadcast_to(a, H.shape).reshape(-1) for a in (3 * r[:, None, None] + k[None, :, None],
+                                                              3 * c[:, None, None] + k[None, None, :]))
+    off = np.repeat(~d, 9)
+    A = sp.coo_matrix((np.concatenate([H.reshape(-1), H.reshape(-1)[off]]),
+                       (np.concatenate([i, j[off]]), np.concatenate([j, i[off]]))), shape=(3 * n, 3 * n)).tocsr()
+    ctx = gpu_ctx
+    M = pkg.SpMat(ctx, ctx.to_device(f), ctx.to_device(r, np.int32), ctx.to_device(c, np.int32), r.size, n, want_f32=True)
+    y = ctx.to_device(np.zeros(3 * n))
+    M.apply_f32_values(1.0, ctx.to_device(x), 0.0, y)
+    M.close()
+    err = (np.abs(y.download() - A @ x) / (abs(A) @ abs(x))).max()
+    print(f"{form} {n} rows: {err:.1e} of the absolute sums")
+    assert err <= 500 * 2.0 ** -53
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32_mas", "fp32_ir"])
 @pytest.mark.parametrize("N,graph", [(9, True), (31, False)])
 def test_default_iteration_folds_the_p_update(pkg, N, precision, graph):
