@@ -57,8 +57,12 @@ namespace {
 //    64 rows    7.1 /  6.5    9.8 /  7.6   18.4 / 14.7   27.1 / 25.5   62.2 / 56.0
 constexpr int kTileLarge = 512, kTileMid = 128, kTileSmall = 64;
 // up to 512 rows one tile holds the whole matrix (no halo); below these counts
-// the smaller tiles
-constexpr int kRowsSmall = 28000, kRowsMid = 80000;
+// the smaller tiles.  With FP32 values two workgroups share a CU, so past 512
+// tiles of 128 rows a second round begins (grid with contacts, 64k and 69k
+// rows: 9.1 and 12.8 us against 12.2 and 13.1 in 512-row tiles; without
+// contacts 8.7 and 12.7 against 11.1 and 11.7); the FP64 products gain up to
+// 80k rows (79k rows: 17.1 against 18.5 us).
+constexpr int kRowsSmall = 28000, kRowsMid = 80000, kRowsMidF32 = 65536;
 constexpr int kSplit = 2;                  // waves per slice (gather form)
 constexpr int kTcap = 4096;                // in-tile transposed slots per tile (LDS)
 constexpr uint32_t kInTile = 0x80000000u;
@@ -1009,7 +1013,7 @@ void FullMatrix::build(hipStream_t s, const double* vals, const int* rows, const
     while (kbits < 31 && (1L << kbits) < (long)n) ++kbits;
     tile_rows = fixed_tiles || n <= kTileLarge ? kTileLarge
                 : n < kRowsSmall               ? kTileSmall
-                                               : (n < kRowsMid ? kTileMid : kTileLarge);
+                                               : (n < (want_f32 ? kRowsMidF32 : kRowsMid) ? kTileMid : kTileLarge);
     n_tiles = (n + tile_rows - 1) / tile_rows;
     const int n_pos = n_tiles * tile_rows;
     n_slices = n_pos / 64;

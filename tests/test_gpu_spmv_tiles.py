@@ -35,7 +35,7 @@ def matrix(n, rng, long_row):
 
 @pytest.mark.parametrize("form", ["halo", "gather"])
 @pytest.mark.parametrize("n,long_row", [(1, False), (65, False), (512, False), (513, False), (1000, True), (27999, False),
-                                        (28000, True), (28127, False), (79999, False), (80000, False), (80513, True)])
+                                        (28000, True), (28127, False), (65535, False), (65537, True), (79999, False), (80000, False), (80513, True)])
 def test_products(pkg, gpu_ctx, monkeypatch, form, n, long_row):
     monkeypatch.setenv("SGIPC_SPMV_GATHER", "1" if form == "gather" else "0")
     rng = np.random.default_rng(n)
