@@ -607,18 +607,26 @@ __global__ __launch_bounds__(256) void k_segment_sum(const double* __restrict__ 
 // workgroup counts its rows in an LDS table, so memory sees one atomic per
 // distinct row and not one per triplet -- and each row is sorted by (column,
 // triplet) on its own: by one wave in registers up to 256 triplets, by one
-// workgroup in LDS up to 16384, and with a longer one the general conversion
-// runs instead.  The sums then read their triplets in exactly the general
-// order, 9 lanes per block (72-byte runs).  16 M triplets (1.47 GB in and
-// out): counting 81 + 103 us, row sorts 147, sums 440 (1.67 GB with the keys
-// at 3.8 TB/s; a large copy reaches 4.75 on this part), 0.9 ms with the index
-// check and the read-back against 1.73 ms for the general conversion.
+// workgroup in LDS up to 2048.  The triplets of longer rows (hubs, the zero
+// blocks of boundary hinges) are sorted together by a radix sort of their own,
+// whose keys hold a row's rank; where they are more than half of all, the
+// general conversion runs instead, and the kernels behind the count leave at
+// once.  The sums then read their triplets in exactly the general order, 9
+// lanes per block (72-byte runs).  16 M triplets (1.47 GB in and out): counting
+// 81 + 103 us, row sorts 147, sums 440 (1.67 GB with the keys at 3.8 TB/s; a
+// large copy reaches 4.75 on this part), 0.87 ms with the index check and the
+// read-back against 1.73 ms for the general conversion.  With long rows: 48 M
+// triplets of a 1024^2 cloth (one row of 65 k) 2.9 ms against 4.7; 1.9 M of
+// two 72^2 sheets (one row of 9 k) 0.42 against 0.42.
 constexpr int kRowTable = 1024;  // slots of the LDS row table
 constexpr int kRowItems = 8;     // triplets per thread
-constexpr int kRowShort = 256, kRowMid = 2048, kRowLong = 16384;
-// words behind the row counts: bad index, a row past kRowLong, rows past
-// kRowShort, rows past kRowMid, unique blocks
-enum { kBad = 0, kTooLong, kNMid, kNLong, kUnique, kRowWords = 8 };
+constexpr int kRowShort = 256, kRowMid = 2048;
+constexpr int kLongShare = 2;
+// words behind the row counts: bad index, rows past kRowShort, rows past
+// kRowMid and their triplets, unique blocks
+enum { kBad = 0, kNMid, kNLong, kLongSum, kUnique, kRowWords = 8 };
+// too many triplets in long rows: the general conversion takes over
+__host__ __device__ inline bool rows_give_up(int long_sum, long n) { return long_sum > n / kLongShare; }
 
 // Counts of the rows (scatter = false), or the triplets' keys (column, then
 // index) to their row's segment (true; start: exclusive scan of the counts,
@@ -629,6 +637,7 @@ __global__ __launch_bounds__(256) void k_rows_bin(const int* __restrict__ rows, 
                                                   const int* __restrict__ start, uint64_t* __restrict__ key)
 {
     __shared__ int srow[kRowTable], scnt[kRowTable], sbase[kRowTable];
+    if (scatter && rows_give_up(words[kLongSum], n)) return;
     for (int i = threadIdx.x; i < kRowTable; i += 256) {
         srow[i] = -1;
         scnt[i] = 0;
@@ -682,6 +691,18 @@ __global__ __launch_bounds__(256) void k_rows_bin(const int* __restrict__ rows, 
     }
 }
 
+// Lists the long rows from the back of the list, each with its place among
+// their triplets.
+__global__ void k_rows_long(int n_rows, const int* __restrict__ cnt, int* __restrict__ words, int* __restrict__ list,
+                            int* __restrict__ base)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n_rows || cnt[r] <= kRowMid) return;
+    const int q = atomicAdd(words + kNLong, 1);
+    list[n_rows - 1 - q] = r;
+    base[q] = atomicAdd(words + kLongSum, cnt[r]);
+}
+
 // One wave per row: its keys sorted in place and its unique columns counted;
 // longer rows are listed.  Bitonic over 64 M elements, element i in lane
 // i % 64, register i / 64; the kernel is bound by its instructions (about 100
@@ -732,10 +753,11 @@ __device__ __forceinline__ int sort_row(uint64_t* __restrict__ seg, int k)
     }
     return u;
 }
-__global__ __launch_bounds__(256) void k_rows_sort(int n_rows, const int* __restrict__ start, uint64_t* __restrict__ key,
-                                                   int* __restrict__ ucnt, int* __restrict__ words,
-                                                   int* __restrict__ list)
+__global__ __launch_bounds__(256) void k_rows_sort(int n_rows, long n, const int* __restrict__ start,
+                                                   uint64_t* __restrict__ key, int* __restrict__ ucnt,
+                                                   int* __restrict__ words, int* __restrict__ list)
 {
+    if (rows_give_up(words[kLongSum], n)) return;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r > n_rows) return;
     if (r == n_rows) {
@@ -752,32 +774,28 @@ __global__ __launch_bounds__(256) void k_rows_sort(int n_rows, const int* __rest
     } else if (k <= kRowShort) {
         u = sort_row<4>(key + b, k);
     } else {
-        // listed from the front (up to kRowMid) or the back of the list
         if (lane == 0) {
             ucnt[r] = 0;  // until its own kernel sets it
             if (k <= kRowMid) list[atomicAdd(words + kNMid, 1)] = r;
-            else list[n_rows - 1 - atomicAdd(words + kNLong, 1)] = r;
-            if (k > kRowLong) words[kTooLong] = 1;
         }
         return;
     }
     if (lane == 0) ucnt[r] = u;
 }
 
-// Longer rows, one workgroup each (a fixed grid walks the list): bitonic sort
-// in LDS, padded to a power of two.
-template <int CAP, int NT>
-__global__ __launch_bounds__(NT) void k_rows_sort_long(int n_rows, const int* __restrict__ start,
-                                                       uint64_t* __restrict__ key, int* __restrict__ ucnt,
-                                                       const int* __restrict__ words, const int* __restrict__ list)
+// Rows past kRowShort, one workgroup each (a fixed grid walks the list):
+// bitonic sort in LDS, padded to a power of two.
+__global__ __launch_bounds__(256) void k_rows_sort_mid(const int* __restrict__ start, uint64_t* __restrict__ key,
+                                                       int* __restrict__ ucnt, const int* __restrict__ words,
+                                                       const int* __restrict__ list)
 {
-    extern __shared__ uint64_t sk[];
+    constexpr int NT = 256;
+    __shared__ uint64_t sk[kRowMid];
     __shared__ int su[NT / 64];
-    const int cnt = words[CAP == kRowMid ? kNMid : kNLong];
+    const int cnt = words[kNMid];
     for (int q = blockIdx.x; q < cnt; q += gridDim.x) {
-        const int r = list[CAP == kRowMid ? q : n_rows - 1 - q];
+        const int r = list[q];
         const int b = start[r], k = start[r + 1] - b;
-        if (k > CAP) continue;  // words[kTooLong]: the general conversion takes over
         int p2 = 2 * kRowShort;
         while (p2 < k) p2 <<= 1;
         for (int i = threadIdx.x; i < p2; i += NT) sk[i] = i < k ? key[b + i] : ~0ull;
@@ -830,7 +848,9 @@ __device__ __forceinline__ double sum_run(const double* __restrict__ tvals, cons
 // Unique blocks of the short rows, one wave per row, 9 lanes per block, 7
 // blocks at a time; a block of more than kSegChunk triplets is the ordered
 // sum of its chunk sums, as in the general conversion.
-__global__ __launch_bounds__(256) void k_rows_sum(const double* __restrict__ tvals, int n_rows,
+// Leaves at once while the long rows' blocks are not counted (n_long: how many
+// are).
+__global__ __launch_bounds__(256) void k_rows_sum(const double* __restrict__ tvals, int n_rows, int n_long,
                                                   const int* __restrict__ start, const uint64_t* __restrict__ key,
                                                   const int* __restrict__ uofs, int cap, double* __restrict__ ovals,
                                                   int* __restrict__ orows, int* __restrict__ ocols,
@@ -838,6 +858,7 @@ __global__ __launch_bounds__(256) void k_rows_sum(const double* __restrict__ tva
 {
     __shared__ uint64_t sm[4][kRowShort];
     __shared__ int hd[4][kRowShort + 1];
+    if (words[kNLong] != n_long) return;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= n_rows) {
         if (r == n_rows && lane == 0) words[kUnique] = uofs[n_rows];
@@ -885,28 +906,28 @@ __global__ __launch_bounds__(256) void k_rows_sum(const double* __restrict__ tva
     }
 }
 
-// Unique blocks of the longer rows, one workgroup per row: the 9-lane groups
+// Unique blocks of the rows past kRowShort, one workgroup per row: the 9-lane groups
 // of all waves take the blocks' chunks in turn (blocks without chunks count
 // as one), then the chunk sums of each block are added in order.
-template <int CAP, int NT>
-__global__ __launch_bounds__(NT) void k_rows_sum_long(const double* __restrict__ tvals, int n_rows,
+__global__ __launch_bounds__(256) void k_rows_sum_mid(const double* __restrict__ tvals, int n_long,
                                                       const int* __restrict__ start, const uint64_t* __restrict__ key,
                                                       const int* __restrict__ uofs, int cap,
                                                       double* __restrict__ ovals, int* __restrict__ orows,
                                                       int* __restrict__ ocols, const int* __restrict__ words,
                                                       const int* __restrict__ list)
 {
-    // chunk sums of the blocks past kSegChunk: their count is below 2 CAP / kSegChunk
-    extern __shared__ double part[];
-    __shared__ int wsum[NT / 64], wblk[NT / 64];
+    constexpr int NT = 256;
+    // chunk sums of the blocks past kSegChunk: their count is below 2 kRowMid / kSegChunk
+    __shared__ double part[9 * (2 * kRowMid / kSegChunk)];
+    __shared__ int head[kRowMid + 1];  // block starts
+    __shared__ int wsum[NT / 64];
     constexpr int kGroups = 7 * (NT / 64);
-    const int cnt = words[CAP == kRowMid ? kNMid : kNLong];
-    int* const head = reinterpret_cast<int*>(part + 9 * (2 * CAP / kSegChunk));  // CAP + 1 block starts
+    if (words[kNLong] != n_long) return;
+    const int cnt = words[kNMid];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int t = blockIdx.x; t < cnt; t += gridDim.x) {
-        const int r = list[CAP == kRowMid ? t : n_rows - 1 - t];
+        const int r = list[t];
         const int b = start[r], k = start[r + 1] - b, o = uofs[r];
-        if (k > CAP) continue;
         // block starts in order
         int u = 0;
         for (int i0 = 0; i0 < k; i0 += NT) {
@@ -974,6 +995,105 @@ __global__ __launch_bounds__(NT) void k_rows_sum_long(const double* __restrict__
             c += nc;
         }
         __syncthreads();
+    }
+}
+
+// ---- long rows: their triplets sorted together
+// rank of the row, column and index of every triplet in one key
+__global__ __launch_bounds__(256) void k_long_pack(int n_rows, const int* __restrict__ list,
+                                                   const int* __restrict__ base, const int* __restrict__ start,
+                                                   const uint64_t* __restrict__ key, int cbits, int ibits,
+                                                   uint64_t* __restrict__ out)
+{
+    const int q = blockIdx.x, r = list[n_rows - 1 - q];
+    const int b = start[r], k = start[r + 1] - b;
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < k; i += gridDim.y * 256) {
+        const uint64_t w = key[b + i];
+        out[base[q] + i] = ((uint64_t)q << (cbits + ibits)) | ((w >> 32) << ibits) | (uint32_t)w;
+    }
+}
+__global__ void k_long_flags(const uint64_t* __restrict__ p, int m, int ibits, int* __restrict__ flag)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < m) flag[t] = (t == 0 || (p[t] >> ibits) != (p[t - 1] >> ibits)) ? 1 : 0;
+}
+// triplet indices in order; per block its first triplet, row rank and column;
+// per row its first block (pos: inclusive scan of the flags)
+// and, added to the 0 there, its block count
+__global__ void k_long_heads(const uint64_t* __restrict__ p, const int* __restrict__ flag, const int* __restrict__ pos,
+                             int m, int n_rows, const int* __restrict__ list, int cbits, int ibits,
+                             int* __restrict__ idx, int* __restrict__ head, int2* __restrict__ id,
+                             int* __restrict__ first, int* __restrict__ ucnt)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= m) return;
+    const uint64_t w = p[t];
+    const int q = (int)(w >> (cbits + ibits)), at = pos[t];
+    idx[t] = (int)(w & ((1ull << ibits) - 1ull));
+    if (flag[t]) {
+        head[at - 1] = t;
+        id[at - 1] = make_int2(q, (int)((w >> ibits) & ((1ull << cbits) - 1ull)));
+    }
+    if (t == 0 || (int)(p[t - 1] >> (cbits + ibits)) != q) {
+        first[q] = at - 1;
+        atomicSub(ucnt + list[n_rows - 1 - q], at - 1);
+    }
+    if (t == m - 1 || (int)(p[t + 1] >> (cbits + ibits)) != q) atomicAdd(ucnt + list[n_rows - 1 - q], at);
+    if (t == m - 1) head[at] = m;
+}
+// Chunk sums of the blocks past kSegChunk, 9 lanes per chunk.  Of 64 sorted
+// triplets, at most one starts a later chunk of a block and one the first
+// chunk of the next such block: places 2 w and 2 w + 1 for triplets 64 w on.
+__device__ __forceinline__ int long_chunk_place(int t, bool is_first) { return 2 * (t / kSegChunk) + (is_first ? 1 : 0); }
+__global__ __launch_bounds__(256) void k_long_chunks(const double* __restrict__ tvals, const int* __restrict__ idx,
+                                                     const int* __restrict__ head, const int* __restrict__ pos, int m,
+                                                     double* __restrict__ part)
+{
+    const int lane = threadIdx.x & 63, e = lane % 9;
+    const long g = (blockIdx.x * 4L + (threadIdx.x >> 6)) * 7 + lane / 9;
+    const long t0 = g / 2 * kSegChunk;
+    if (lane == 63 || t0 >= m) return;
+    const bool is_first = (g & 1) != 0;
+    const int t1 = (int)min(t0 + kSegChunk, (long)m);
+    const int u = pos[is_first ? t1 - 1 : t0] - 1;  // the last block that starts here, or the one that t0 lies in
+    const int b = head[u], end = head[u + 1];
+    const int c = is_first ? b : b + ((int)t0 - b + kSegChunk - 1) / kSegChunk * kSegChunk;
+    if (end - b <= kSegChunk || c < t0 || c >= min(t1, end) || is_first != (c == b)) return;
+    double s = 0.0;
+#pragma unroll 4
+    for (int t = c; t < min(c + kSegChunk, end); ++t) s += tvals[9 * (long)idx[t] + e];
+    part[9 * g + e] = s;
+}
+// 9 lanes per block, 7 blocks per wave: its triplets in order, or its chunk
+// sums in order
+__global__ __launch_bounds__(256) void k_long_sum(const double* __restrict__ tvals, const int* __restrict__ idx,
+                                                  const int* __restrict__ head, const int2* __restrict__ id,
+                                                  const int* __restrict__ first, const int* __restrict__ n_blocks,
+                                                  int n_rows, const int* __restrict__ list,
+                                                  const double* __restrict__ part, const int* __restrict__ uofs,
+                                                  int cap, double* __restrict__ ovals, int* __restrict__ orows,
+                                                  int* __restrict__ ocols)
+{
+    const int lane = threadIdx.x & 63, e = lane % 9;
+    const long u = (blockIdx.x * 4L + (threadIdx.x >> 6)) * 7 + lane / 9;
+    if (lane == 63 || u >= *n_blocks) return;
+    const int2 w = id[u];
+    const int r = list[n_rows - 1 - w.x];
+    const long o = uofs[r] + (u - first[w.x]);
+    if (o >= cap) return;
+    double s = 0.0;
+    const int b = head[u], end = head[u + 1];
+    if (end - b > kSegChunk) {
+#pragma unroll 4
+        for (int t = b; t < end; t += kSegChunk) s += part[9L * long_chunk_place(t, t == b) + e];
+    } else {
+#pragma unroll 4
+        for (int t = b; t < end; ++t) s += tvals[9 * (long)idx[t] + e];
+    }
+    ovals[9 * o + e] = s;
+    if (e == 0) {
+        orows[o] = r;
+        ocols[o] = w.y;
     }
 }
 
@@ -1136,6 +1256,7 @@ bool Converter::convert_rows(hipStream_t s, const double* tvals, const int* trow
     row_ucnt_.reserve(R + 1);
     row_uofs_.reserve(R + 1);
     row_list_.reserve(R > 0 ? R : 1);
+    row_base_.reserve(n / kRowMid + 1);
     keys_.reserve(n);
     int* const cnt = row_cnt_.get();
     int* const words = cnt + R + 1;
@@ -1146,68 +1267,101 @@ bool Converter::convert_rows(hipStream_t s, const double* tvals, const int* trow
     const int gb = (int)((n + 256 * kRowItems - 1) / (256 * kRowItems));
     k_rows_bin<false><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, nullptr, nullptr);
     SGIPC_LAUNCH_CHECK();
+    if (n > kRowMid) {
+        k_rows_long<<<g256(R), 256, 0, s>>>(n_rows, cnt, words, row_list_.get(), row_base_.get());
+        SGIPC_LAUNCH_CHECK();
+    }
     SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, cnt, row_start_.get(), 0, (size_t)(R + 1),
                                       rocprim::plus<int>(), s));
     k_rows_bin<true><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, row_start_.get(), keys_.get());
     SGIPC_LAUNCH_CHECK();
     const int gr = (int)((R + 1 + 3) / 4);
-    k_rows_sort<<<gr, 256, 0, s>>>(n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+    k_rows_sort<<<gr, 256, 0, s>>>(n_rows, n, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
     SGIPC_LAUNCH_CHECK();
-    // the longer rows: grids that walk the lists (their lengths stay on the device)
-    const int g_mid = (int)std::min<long>(1024, n / kRowShort), g_long = (int)std::min<long>(256, n / kRowMid);
+    // rows past kRowShort: a grid that walks the list (its length stays on the device)
+    const int g_mid = (int)std::min<long>(1024, n / kRowShort);
     if (g_mid > 0) {
-        k_rows_sort_long<kRowMid, 256><<<g_mid, 256, kRowMid * sizeof(uint64_t), s>>>(
-            n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+        k_rows_sort_mid<<<g_mid, 256, 0, s>>>(row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
         SGIPC_LAUNCH_CHECK();
     }
-    auto sum_lds = [](int cap) { return 9 * sizeof(double) * (2 * cap / kSegChunk) + sizeof(int) * (cap + 1); };
-    if (g_long > 0) {
-        // more LDS than a launch gets by default (set on the current device)
-        SGIPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rows_sort_long<kRowLong, 1024>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, kRowLong * sizeof(uint64_t)));
-        SGIPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_rows_sum_long<kRowLong, 1024>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sum_lds(kRowLong)));
-        k_rows_sort_long<kRowLong, 1024><<<g_long, 1024, kRowLong * sizeof(uint64_t), s>>>(
-            n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+    // the blocks' places and sums, but those of n_long long rows
+    auto sums = [&](int n_long) {
+        SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, row_ucnt_.get(), row_uofs_.get(), 0, (size_t)(R + 1),
+                                          rocprim::plus<int>(), s));
+        k_rows_sum<<<gr, 256, 0, s>>>(tvals, n_rows, n_long, row_start_.get(), keys_.get(), row_uofs_.get(), capacity,
+                                      ovals, orows, ocols, words);
         SGIPC_LAUNCH_CHECK();
-    }
-    SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, row_ucnt_.get(), row_uofs_.get(), 0, (size_t)(R + 1),
-                                      rocprim::plus<int>(), s));
-    k_rows_sum<<<gr, 256, 0, s>>>(tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals,
-                                  orows, ocols, words);
-    SGIPC_LAUNCH_CHECK();
-    if (g_mid > 0) {
-        k_rows_sum_long<kRowMid, 256><<<g_mid, 256, sum_lds(kRowMid), s>>>(
-            tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals, orows, ocols, words,
-            row_list_.get());
-        SGIPC_LAUNCH_CHECK();
-    }
-    if (g_long > 0) {
-        k_rows_sum_long<kRowLong, 1024><<<g_long, 1024, sum_lds(kRowLong), s>>>(
-            tvals, n_rows, row_start_.get(), keys_.get(), row_uofs_.get(), capacity, ovals, orows, ocols, words,
-            row_list_.get());
-        SGIPC_LAUNCH_CHECK();
-    }
+        if (g_mid > 0) {
+            k_rows_sum_mid<<<g_mid, 256, 0, s>>>(tvals, n_long, row_start_.get(), keys_.get(), row_uofs_.get(),
+                                                 capacity, ovals, orows, ocols, words, row_list_.get());
+            SGIPC_LAUNCH_CHECK();
+        }
+    };
     int h[kRowWords];
-    SGIPC_HIP(hipMemcpyAsync(h, words, sizeof(h), hipMemcpyDeviceToHost, s));
-    SGIPC_HIP(hipStreamSynchronize(s));
+    auto read_words = [&] {
+        SGIPC_HIP(hipMemcpyAsync(h, words, sizeof(h), hipMemcpyDeviceToHost, s));
+        SGIPC_HIP(hipStreamSynchronize(s));
+    };
+    sums(0);
+    read_words();
     SGIPC_CHECK(h[kBad] == 0, SGIPC_BAD_INDEX,
                 "triplet with row > col, a negative index or an index beyond the bound");
-    if (h[kTooLong]) return false;
+    const int n_long = h[kNLong], m = h[kLongSum];
+    if (n_long > 0) {
+        const int qbits = index_bits(n_long), cbits = index_bits(n_rows), ibits = index_bits((int)n);
+        if (rows_give_up(m, n) || qbits + cbits + ibits > 64) return false;
+        skeys_.reserve(2L * m);
+        idx_.reserve(m);
+        flag_.reserve(m);
+        pos_.reserve(m);
+        head_.reserve(m + 1L);
+        long_id_.reserve(m);
+        row_first_.reserve(n_long);
+        uint64_t* const packed = skeys_.get();
+        uint64_t* const sorted = packed + m;
+        size_t n1 = 0, n2 = 0;
+        SGIPC_HIP(rocprim::radix_sort_keys(nullptr, n1, packed, sorted, (size_t)m, 0, qbits + cbits + ibits, s));
+        SGIPC_HIP(rocprim::inclusive_scan(nullptr, n2, flag_.get(), pos_.get(), (size_t)m, rocprim::plus<int>(), s));
+        temp_.reserve(std::max(std::max(n1, n2), need));
+        const unsigned gy = (unsigned)std::min<long>(64, m / n_long / 1024 + 1);
+        k_long_pack<<<dim3(n_long, gy), 256, 0, s>>>(n_rows, row_list_.get(), row_base_.get(), row_start_.get(),
+                                                     keys_.get(), cbits, ibits, packed);
+        SGIPC_LAUNCH_CHECK();
+        SGIPC_HIP(rocprim::radix_sort_keys(temp_.get(), n1, packed, sorted, (size_t)m, 0, qbits + cbits + ibits, s));
+        k_long_flags<<<g256(m), 256, 0, s>>>(sorted, m, ibits, flag_.get());
+        SGIPC_LAUNCH_CHECK();
+        SGIPC_HIP(rocprim::inclusive_scan(temp_.get(), n2, flag_.get(), pos_.get(), (size_t)m, rocprim::plus<int>(), s));
+        k_long_heads<<<g256(m), 256, 0, s>>>(sorted, flag_.get(), pos_.get(), m, n_rows, row_list_.get(), cbits, ibits,
+                                             idx_.get(), head_.get(), long_id_.get(), row_first_.get(), row_ucnt_.get());
+        SGIPC_LAUNCH_CHECK();
+        sums(n_long);
+        // chunk sums over the packed keys (2 of 9 doubles for every 64 triplets)
+        double* const part = reinterpret_cast<double*>(packed);
+        const long places = 2 * ((m + (long)kSegChunk - 1) / kSegChunk);
+        k_long_chunks<<<(int)((places + 27) / 28), 256, 0, s>>>(tvals, idx_.get(), head_.get(), pos_.get(), m, part);
+        SGIPC_LAUNCH_CHECK();
+        k_long_sum<<<(m + 27) / 28, 256, 0, s>>>(tvals, idx_.get(), head_.get(), long_id_.get(), row_first_.get(),
+                                                 pos_.get() + (m - 1), n_rows, row_list_.get(), part, row_uofs_.get(),
+                                                 capacity, ovals, orows, ocols);
+        SGIPC_LAUNCH_CHECK();
+        read_words();
+    }
     *unique = h[kUnique];
     SGIPC_CHECK(*unique <= capacity, SGIPC_CAPACITY, "unique block count exceeds the output capacity");
     return true;
 }
 
 int Converter::convert(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n,
-                       int index_bound, double* ovals, int* orows, int* ocols, int capacity)
+                       int index_bound, double* ovals, int* orows, int* ocols, int capacity, bool long_rows)
 {
     if (n <= 0) return 0;
     SGIPC_CHECK(n < (1L << 31), SGIPC_CAPACITY, "too many triplets");
-    // By rows unless the rows are so few that they must be long (then their
-    // sorts would leave the chip idle), or so many that their tables outweigh
-    // the triplets, or one proves too long.
-    if (index_bound < (1L << 31) - 8 && n <= 2048L * index_bound && index_bound <= 4 * n + 4096 &&
+    // By rows unless they are longer on average than a wave sorts (3.2 M
+    // triplets in 2133 rows: 0.92 ms against 0.47), or so many that their
+    // tables outweigh the triplets, or the caller or the count says that much
+    // lies in long rows (0.35 M triplets, a third of them in 8 rows: 0.70 ms
+    // by rows against 0.34).
+    if (!long_rows && index_bound < (1L << 31) - 8 && n <= 256L * index_bound && index_bound <= 4 * n + 4096 &&
         convert_rows(s, tvals, trows, tcols, n, index_bound, ovals, orows, ocols, capacity, &last_unique))
         return last_unique;
     keys_.reserve(n);

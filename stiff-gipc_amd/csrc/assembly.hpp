@@ -52,9 +52,10 @@ int convert_into(hipStream_t s, const ConvertScratch& w, const double* tvals, co
 class Converter {
   public:
     // Returns the unique block count; throws SGIPC_CAPACITY / SGIPC_BAD_INDEX.
-    // index_bound: every row/col is < index_bound.
+    // index_bound: every row/col is < index_bound.  long_rows: a hint that many
+    // triplets lie in rows of thousands (the results do not depend on it).
     int convert(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n, int index_bound,
-                double* ovals, int* orows, int* ocols, int capacity);
+                double* ovals, int* orows, int* ocols, int capacity, bool long_rows = false);
     int max_index(hipStream_t s, const int* rows, const int* cols, long n);
     static int index_bits(int bound);
     // unique block count of the last convert, also when it threw
@@ -62,11 +63,12 @@ class Converter {
     int last_unique = 0;
 
   private:
-    // The conversion by row counting and per-row sorts; false when a row is
-    // too long for it (nothing of use written then).
+    // The conversion by row counting and per-row sorts; false when too much
+    // lies in long rows (nothing of use written then).
     bool convert_rows(hipStream_t s, const double* tvals, const int* trows, const int* tcols, long n, int n_rows,
                       double* ovals, int* orows, int* ocols, int capacity, int* unique);
-    DevBuf<int> row_cnt_, row_start_, row_ucnt_, row_uofs_, row_list_;
+    DevBuf<int> row_cnt_, row_start_, row_ucnt_, row_uofs_, row_list_, row_base_, row_first_;
+    DevBuf<int2> long_id_;
     DevBuf<uint64_t> keys_, skeys_;
     DevBuf<int> idx_, sidx_, flag_, pos_, head_, scratch_int_;
     DevBuf<unsigned char> temp_;

@@ -776,8 +776,10 @@ int system_solve(sgipc_system* sys, const double* b, double* x, double* grad, co
             }
         });
         try {
+            // a pair puts about 7 triplets into the first row of its body
+            const bool long_rows = nb > 0 && 7L * d.n_pairs > 2048L * nb;
             sys->nnz = sys->conv.convert(s, sys->tvals.get(), sys->trows.get(), sys->tcols.get(), off, sys->n_sys,
-                                         sys->bvals.get(), sys->brows.get(), sys->bcols.get(), sys->capacity);
+                                         sys->bvals.get(), sys->brows.get(), sys->bcols.get(), sys->capacity, long_rows);
         } catch (...) {
             hier.join();
             throw;

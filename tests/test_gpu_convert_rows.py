@@ -1,8 +1,9 @@
 """The conversion by row counting at the row lengths where its paths change
-(a wave's 64, 128 and 256 triplets, a workgroup's 2048 and 16384, the general
-conversion past that), with blocks of more and fewer than 64 triplets: values
-bit-exact against the oracle (the order of the sums is part of the result),
-indices, counts and status codes equal."""
+(a wave's 64, 128 and 256 triplets, a workgroup's 2048, the common sort of the
+longer rows, the general conversion when these hold more than half of the
+triplets), with blocks of more and fewer than 64 triplets: values bit-exact
+against the oracle (the order of the sums is part of the result), indices,
+counts and status codes equal."""
 import ctypes
 
 import numpy as np
@@ -38,6 +39,12 @@ ROWS = {
     "long": ([16383, 16384, 100], 5000),
     "too_long": ([16385, 30, 0, 9], 300),
     "few_rows": ([9000], 3),
+    "some_long": ([2049, 30, 5000, 2048] + [40] * 2000 + [3000], 700),
+    "long_one_block": ([9000] + [90] * 1000, 1),
+    "long_last": ([20] * 3000 + [4097, 2500], 30000),
+    "share_below": ([20000] + [25] * 800, 100),
+    "share_above": ([20001] + [25] * 800, 100),
+    "many_long": ([2100] * 40 + [64] * 12000, 3000),
     "many_short": (list(np.random.default_rng(1).integers(0, 90, 3000)), 12),
 }
 
