@@ -467,9 +467,10 @@ __global__ __launch_bounds__(256) void k_bwd_gather(int n, const int* __restrict
 
 // First layer: dW_in[g][c] partial = sum_rows X[row][g] (G + dU_self)[row][c]
 //                                    + (Ahat X)[row][g] dU_nb[row][c]
-// over 256-row chunks; Ahat X as the forward pass left it (forming it again
-// from the graph for every channel took 347 us on 16 samples of 8k nodes,
-// reading it 78 us).
+// over the 96 rows of 32 nodes, a wave's 8 nodes (24 rows) in FP32 and the
+// partials in FP64: longer FP32 chains lose what stands behind a large term.
+// Ahat X as the forward pass left it (forming it again from the graph for
+// every channel took 347 us on 16 samples of 8k nodes, reading it 81 us).
 __global__ __launch_bounds__(256) void k_bwd_win(long rows, const float* __restrict__ X, const float* __restrict__ AX,
                                                  const float* __restrict__ G, const float* __restrict__ dU,
                                                  float* __restrict__ part)
@@ -478,11 +479,11 @@ __global__ __launch_bounds__(256) void k_bwd_win(long rows, const float* __restr
     const int t = threadIdx.x;
     const int ch = t & 63;
     const int wv = t >> 6;
-    const long r0 = (long)blockIdx.x * 256;
+    const long r0 = (long)blockIdx.x * kRows;
     float acc[3] = {0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int k = wv; k < 256; k += 4) {
-        const long row = r0 + k;
+#pragma unroll
+    for (int k = 0; k < kRows / 4; ++k) {
+        const long row = r0 + 3 * (wv + 4 * (k / 3)) + k % 3;
         if (row >= rows) break;
         const float gs = G[row * C + ch] + dU[row * 2 * C + ch];
         const float gn = dU[row * 2 * C + C + ch];
@@ -826,7 +827,7 @@ double Mpnn::loss_grad(hipStream_t st, const CoarseGraph& g, const float* X, con
     const int gl = g256(nodes);
     const int n_dec = g256(rows);
     const int n_dw = (int)((rows + kDwRows - 1) / kDwRows);
-    const int n_win = g256(rows);
+    const int n_win = (int)((rows + kRows - 1) / kRows);
     const long part_need = std::max({(long)gl, (long)n_dec * C, (long)n_dw * 2 * C * C, (long)n_win * 3 * C});
     part_.reserve(part_need);
     DevBuf<double>& lp = lpart_;
