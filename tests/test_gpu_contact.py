@@ -1,4 +1,4 @@
-"""Contact detection (LBVH) and the barrier of every pair type on the GPU,
+"""Contact detection and the barrier of every pair type on the GPU,
 against the oracle through the C ABI.
 
 Tolerances:
@@ -74,7 +74,8 @@ def test_detection_large_sheet_properties(pkg, orc, gpu_ctx):
     e = orc.barrier_energy(geo.x, pr, geo.dhat ** 2, geo.kappa)
     assert np.isfinite(e) and e > 0
     print(f"sheets256: {n} pairs, barrier energy {e:.3e}")
-    assert n > 4 * geo.n
+    # 48^2 sheets (against the oracle above) hold 13.3 pairs a vertex, and larger ones lose less at their borders
+    assert n > 13.3 * geo.n
 
 
 @pytest.mark.parametrize("N", [12, 32])
