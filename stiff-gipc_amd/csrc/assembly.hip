@@ -610,23 +610,20 @@ __global__ __launch_bounds__(256) void k_segment_sum(const double* __restrict__ 
 // workgroup in LDS up to 2048.  The triplets of longer rows (hubs, the zero
 // blocks of boundary hinges) are sorted together by a radix sort of their own,
 // whose keys hold a row's rank; where they are more than half of all, the
-// general conversion runs instead, and the kernels behind the count leave at
-// once.  The sums then read their triplets in exactly the general order, 9
-// lanes per block (72-byte runs).  16 M triplets (1.47 GB in and out): counting
-// 81 + 103 us, row sorts 147, sums 440 (1.67 GB with the keys at 3.8 TB/s; a
-// large copy reaches 4.75 on this part), 0.87 ms with the index check and the
-// read-back against 1.73 ms for the general conversion.  With long rows: 48 M
+// general conversion runs instead.  The sums then read their triplets in
+// exactly the general order, 9 lanes per block (72-byte runs).  16 M triplets
+// (1.47 GB in and out): counting 81 + 103 us, row sorts 147, sums 440 (1.67 GB
+// with the keys at 3.8 TB/s; a large copy reaches 4.75 on this part), 0.87 ms
+// with the index check and the read-back against 1.73 ms for the general
+// conversion.  With long rows: 48 M
 // triplets of a 1024^2 cloth (one row of 65 k) 2.9 ms against 4.7; 1.9 M of
 // two 72^2 sheets (one row of 9 k) 0.42 against 0.42.
 constexpr int kRowTable = 1024;  // slots of the LDS row table
 constexpr int kRowItems = 8;     // triplets per thread
 constexpr int kRowShort = 256, kRowMid = 2048;
-constexpr int kLongShare = 2;
 // words behind the row counts: bad index, rows past kRowShort, rows past
 // kRowMid and their triplets, unique blocks
 enum { kBad = 0, kNMid, kNLong, kLongSum, kUnique, kRowWords = 8 };
-// too many triplets in long rows: the general conversion takes over
-__host__ __device__ inline bool rows_give_up(int long_sum, long n) { return long_sum > n / kLongShare; }
 
 // Counts of the rows (scatter = false), or the triplets' keys (column, then
 // index) to their row's segment (true; start: exclusive scan of the counts,
@@ -637,7 +634,6 @@ __global__ __launch_bounds__(256) void k_rows_bin(const int* __restrict__ rows, 
                                                   const int* __restrict__ start, uint64_t* __restrict__ key)
 {
     __shared__ int srow[kRowTable], scnt[kRowTable], sbase[kRowTable];
-    if (scatter && rows_give_up(words[kLongSum], n)) return;
     for (int i = threadIdx.x; i < kRowTable; i += 256) {
         srow[i] = -1;
         scnt[i] = 0;
@@ -691,18 +687,6 @@ __global__ __launch_bounds__(256) void k_rows_bin(const int* __restrict__ rows, 
     }
 }
 
-// Lists the long rows from the back of the list, each with its place among
-// their triplets.
-__global__ void k_rows_long(int n_rows, const int* __restrict__ cnt, int* __restrict__ words, int* __restrict__ list,
-                            int* __restrict__ base)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rows || cnt[r] <= kRowMid) return;
-    const int q = atomicAdd(words + kNLong, 1);
-    list[n_rows - 1 - q] = r;
-    base[q] = atomicAdd(words + kLongSum, cnt[r]);
-}
-
 // One wave per row: its keys sorted in place and its unique columns counted;
 // longer rows are listed.  Bitonic over 64 M elements, element i in lane
 // i % 64, register i / 64; the kernel is bound by its instructions (about 100
@@ -753,11 +737,10 @@ __device__ __forceinline__ int sort_row(uint64_t* __restrict__ seg, int k)
     }
     return u;
 }
-__global__ __launch_bounds__(256) void k_rows_sort(int n_rows, long n, const int* __restrict__ start,
-                                                   uint64_t* __restrict__ key, int* __restrict__ ucnt,
-                                                   int* __restrict__ words, int* __restrict__ list)
+__global__ __launch_bounds__(256) void k_rows_sort(int n_rows, const int* __restrict__ start, uint64_t* __restrict__ key,
+                                                   int* __restrict__ ucnt, int* __restrict__ words,
+                                                   int* __restrict__ list, int* __restrict__ base)
 {
-    if (rows_give_up(words[kLongSum], n)) return;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r > n_rows) return;
     if (r == n_rows) {
@@ -774,9 +757,17 @@ __global__ __launch_bounds__(256) void k_rows_sort(int n_rows, long n, const int
     } else if (k <= kRowShort) {
         u = sort_row<4>(key + b, k);
     } else {
+        // listed from the front (up to kRowMid) or the back of the list, there
+        // with its place among the long rows' triplets
         if (lane == 0) {
             ucnt[r] = 0;  // until its own kernel sets it
-            if (k <= kRowMid) list[atomicAdd(words + kNMid, 1)] = r;
+            if (k <= kRowMid) {
+                list[atomicAdd(words + kNMid, 1)] = r;
+            } else {
+                const int q = atomicAdd(words + kNLong, 1);
+                list[n_rows - 1 - q] = r;
+                base[q] = atomicAdd(words + kLongSum, k);
+            }
         }
         return;
     }
@@ -1267,16 +1258,13 @@ bool Converter::convert_rows(hipStream_t s, const double* tvals, const int* trow
     const int gb = (int)((n + 256 * kRowItems - 1) / (256 * kRowItems));
     k_rows_bin<false><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, nullptr, nullptr);
     SGIPC_LAUNCH_CHECK();
-    if (n > kRowMid) {
-        k_rows_long<<<g256(R), 256, 0, s>>>(n_rows, cnt, words, row_list_.get(), row_base_.get());
-        SGIPC_LAUNCH_CHECK();
-    }
     SGIPC_HIP(rocprim::exclusive_scan(temp_.get(), need, cnt, row_start_.get(), 0, (size_t)(R + 1),
                                       rocprim::plus<int>(), s));
     k_rows_bin<true><<<gb, 256, 0, s>>>(trows, tcols, n, n_rows, cnt, words, row_start_.get(), keys_.get());
     SGIPC_LAUNCH_CHECK();
     const int gr = (int)((R + 1 + 3) / 4);
-    k_rows_sort<<<gr, 256, 0, s>>>(n_rows, n, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get());
+    k_rows_sort<<<gr, 256, 0, s>>>(n_rows, row_start_.get(), keys_.get(), row_ucnt_.get(), words, row_list_.get(),
+                                   row_base_.get());
     SGIPC_LAUNCH_CHECK();
     // rows past kRowShort: a grid that walks the list (its length stays on the device)
     const int g_mid = (int)std::min<long>(1024, n / kRowShort);
@@ -1309,7 +1297,7 @@ bool Converter::convert_rows(hipStream_t s, const double* tvals, const int* trow
     const int n_long = h[kNLong], m = h[kLongSum];
     if (n_long > 0) {
         const int qbits = index_bits(n_long), cbits = index_bits(n_rows), ibits = index_bits((int)n);
-        if (rows_give_up(m, n) || qbits + cbits + ibits > 64) return false;
+        if (m > n / 2 || qbits + cbits + ibits > 64) return false;
         skeys_.reserve(2L * m);
         idx_.reserve(m);
         flag_.reserve(m);
@@ -1356,12 +1344,13 @@ int Converter::convert(hipStream_t s, const double* tvals, const int* trows, con
 {
     if (n <= 0) return 0;
     SGIPC_CHECK(n < (1L << 31), SGIPC_CAPACITY, "too many triplets");
-    // By rows unless they are longer on average than a wave sorts (3.2 M
-    // triplets in 2133 rows: 0.92 ms against 0.47), or so many that their
-    // tables outweigh the triplets, or the caller or the count says that much
-    // lies in long rows (0.35 M triplets, a third of them in 8 rows: 0.70 ms
-    // by rows against 0.34).
-    if (!long_rows && index_bound < (1L << 31) - 8 && n <= 256L * index_bound && index_bound <= 4 * n + 4096 &&
+    // By rows unless the rows are so few that they must be long, or so many
+    // that their tables outweigh the triplets, or the caller or the count says
+    // that much lies in long rows (0.35 M triplets, a third of them in 8 rows:
+    // 0.70 ms by rows, each long one sorted by a workgroup, against 0.34).
+    // Coarse levels with 400 to 1600 triplets a row: 44k to 1.4 M of them
+    // 0.12 .. 0.28 ms against 0.21 .. 0.36, 5.6 M 0.68 against 0.70.
+    if (!long_rows && index_bound < (1L << 31) - 8 && n <= 2048L * index_bound && index_bound <= 4 * n + 4096 &&
         convert_rows(s, tvals, trows, tcols, n, index_bound, ovals, orows, ocols, capacity, &last_unique))
         return last_unique;
     keys_.reserve(n);
