@@ -182,7 +182,11 @@ __device__ __forceinline__ void rank1_upper(double acc[78], const double g[12], 
 // alone change nothing (0.90).  The modes keep the order of their sums:
 // forming the blocks in the singular bases (U M_ab U^T) took 0.41 ms but
 // raised the error against 64 bits from 1.2e-15 to 1.4e-15.
-constexpr int kTetThreads = 128;
+// kFew: below kTetFew tets the chip is not full and a thread's own stores and
+// atomics are over before the workgroup has met (with the launch: 750 and 13k
+// tets 42 and 45 us against 46 and 48; 41k 63 against 52).
+constexpr int kTetThreads = 128, kTetFew = 20000;
+template <bool kFew>
 __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const double* __restrict__ x,
                                                  const uint4* __restrict__ tets, const double* __restrict__ dm_inv,
                                                  const double* __restrict__ vol, const double* __restrict__ mu_,
@@ -190,10 +194,11 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
                                                  double* __restrict__ grad, double* __restrict__ tvals,
                                                  int* __restrict__ trows, int* __restrict__ tcols)
 {
-    __shared__ double stage[kTetThreads / 64][64 * 18];
-    __shared__ double forces[kTetThreads][13];
-    __shared__ VertexSums<256> sums;
-    if (grad) sums.init();
+    __shared__ double stage[kFew ? 1 : kTetThreads / 64][kFew ? 1 : 64 * 18];
+    __shared__ double forces[kFew ? 1 : kTetThreads][13];
+    __shared__ VertexSums<kFew ? 2 : 256> sums;
+    if constexpr (!kFew)
+        if (grad) sums.init();
     const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
     const bool act = t0 < n_tets;
     const int t = act ? t0 : n_tets - 1;  // spare lanes repeat the last tet and write nothing
@@ -251,7 +256,11 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
                 double s = 0.0;
 #pragma unroll
                 for (int j = 0; j < 3; ++j) s += (mu * F[d][j] + c * cof[d][j]) * D[a][j];
-                if (act) forces[threadIdx.x][3 * a + d] = scale * s;
+                if constexpr (kFew) {
+                    if (act) atomic_add(grad + 3 * (long)vid[a] + d, scale * s);
+                } else {
+                    if (act) forces[threadIdx.x][3 * a + d] = scale * s;
+                }
             }
     }
 
@@ -315,6 +324,29 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
     }
     // 10 upper blocks, local (ii <= jj), stored at (min, max) of the global
     // ids: transposed when the ids are in the other order
+    constexpr int kI[10] = {0, 0, 0, 0, 1, 1, 1, 2, 2, 3}, kJ[10] = {0, 1, 2, 3, 1, 2, 3, 2, 3, 3};
+    if constexpr (kFew) {
+        if (!act) return;
+#pragma unroll
+        for (int k = 0; k < 10; ++k) {
+            const long at = 10 * (long)t + k;
+            const int ii = kI[k], jj = kJ[k];
+            const int a = (int)vid[ii] + hess_offset, b = (int)vid[jj] + hess_offset;
+            const bool keep = a <= b;
+            trows[at] = min(a, b);
+            tcols[at] = max(a, b);
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc) {
+                    const int R = 3 * ii + r, C = 3 * jj + cc, R2 = 3 * jj + r, C2 = 3 * ii + cc;
+                    const double hv = acc[R <= C ? up12(R, C) : up12(C, R)];
+                    const double ht = acc[R2 <= C2 ? up12(R2, C2) : up12(C2, R2)];
+                    tvals[9 * at + cc * 3 + r] = scale * (keep ? hv : ht);
+                }
+        }
+        return;
+    }
     const int lane = threadIdx.x & 63;
     double* const st = stage[threadIdx.x >> 6];
     const long w0 = (long)blockIdx.x * blockDim.x + (threadIdx.x & ~63);  // the wave's first tet
@@ -326,7 +358,6 @@ __global__ __launch_bounds__(kTetThreads) void k_tet_snh(int n_tets, const doubl
         const unsigned e = lane + 64 * i;
         ofs[i] = 90u * (e / 18u) + e % 18u;
     }
-    constexpr int kI[10] = {0, 0, 0, 0, 1, 1, 1, 2, 2, 3}, kJ[10] = {0, 1, 2, 3, 1, 2, 3, 2, 3, 3};
 #pragma unroll
     for (int k0 = 0; k0 < 10; k0 += 2) {
 #pragma unroll
@@ -1123,8 +1154,10 @@ void launch_tet_snh(hipStream_t s, int n_tets, const double* x, const uint32_t* 
                     double* grad, double* tvals, int* trows, int* tcols)
 {
     if (n_tets <= 0) return;
-    k_tet_snh<<<(n_tets + kTetThreads - 1) / kTetThreads, kTetThreads, 0, s>>>(n_tets, x, reinterpret_cast<const uint4*>(tets), dm_inv, vol, mu,
-                                                   lam, dt * dt, hess_offset, grad, tvals, trows, tcols);
+    const auto kernel = n_tets < kTetFew ? &k_tet_snh<true> : &k_tet_snh<false>;
+    kernel<<<(n_tets + kTetThreads - 1) / kTetThreads, kTetThreads, 0, s>>>(
+        n_tets, x, reinterpret_cast<const uint4*>(tets), dm_inv, vol, mu, lam, dt * dt, hess_offset, grad, tvals, trows,
+        tcols);
     SGIPC_LAUNCH_CHECK();
 }
 

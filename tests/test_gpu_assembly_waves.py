@@ -1,7 +1,7 @@
-"""Element kernels that pass their blocks through LDS wave by wave, at element
-counts around a wave (64) and a workgroup (128), with vertex ids in any order
-(blocks stored transposed) and gradients whose vertices collide in the
-workgroup's table: against the oracle within 1e-10 of each element's largest
+"""The tet kernel on both sides of the count from which it passes its blocks
+through LDS wave by wave (20,000), at counts around a wave (64) and a workgroup
+(128), with vertex ids in any order (blocks stored transposed) and gradients
+whose vertices collide in the workgroup's table: against the oracle within 1e-10 of each element's largest
 entry (the element arithmetic's rounding), the gradient within 1e-12
 relative, with indices exact."""
 import dataclasses
@@ -12,7 +12,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m", [1, 63, 64, 65, 127, 128, 129, 300])
+@pytest.mark.parametrize("m", [1, 63, 64, 65, 127, 128, 129, 300, 19999, 20000, 20031, 20032, 20033, 20096, 20097])
 @pytest.mark.parametrize("spread", [False, True])
 def test_tets(pkg, orc, gpu_ctx, m, spread):
     base = pkg.scenes.tet_grid_scene("waves", 6, E_loguniform=(1e4, 1e9))
@@ -23,7 +23,7 @@ def test_tets(pkg, orc, gpu_ctx, m, spread):
     n = 100_000 if spread else base.n
     x = np.zeros((n, 3))
     x[ids[new]] = base.x
-    pick = rng.choice(base.n_tets, m, replace=False)
+    pick = rng.choice(base.n_tets, m, replace=m > base.n_tets)
     tets = ids[new][base.tets[pick]].astype(np.int32)
     part = [np.ascontiguousarray(a[pick]) for a in (base.dm_inv, base.vol, base.mu, base.lam)]
     scene = dataclasses.replace(base, x=x, tets=tets, **dict(zip(("dm_inv", "vol", "mu", "lam"), part)))
