@@ -881,7 +881,7 @@ struct Vec4Of<double> {
 // Row block rb of Minv r for a domain staged in LDS (upper 3x3 blocks, column
 // major inside a block; r in sR): thread (rb, g) sums the column blocks
 // cb = g, g+G, ..., and the G partials of a row, held by adjacent lanes, are
-// added by shuffles in a fixed order.  Every lane ends with its row's sum.
+// added by DPP (group_sum) in a fixed order.  Every lane ends with its row's sum.
 template <int B, typename TS>
 __device__ __forceinline__ void domain_product(const TS* __restrict__ sM, const TS* __restrict__ sR, int rb, int g,
                                                TS& z0, TS& z1, TS& z2)
@@ -976,7 +976,7 @@ __global__ __launch_bounds__(256) void k_half_level0(const float* __restrict__ m
 // All loads of the domain's inverse blocks are issued before any LDS store so
 // the whole 19/38 KB domain is in flight at once.  Thread (rb, g) forms the
 // partial product of block row rb with the column blocks cb = g, g+G, ...;
-// the G partials of a row sit in adjacent lanes and are summed by shuffles in
+// the G partials of a row sit in adjacent lanes and are summed by DPP in
 // a fixed order.
 template <int B, typename TS>
 __global__ __launch_bounds__(256) void k_local_solve(const int* __restrict__ done, const TS* __restrict__ minv,

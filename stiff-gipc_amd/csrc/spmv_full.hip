@@ -50,11 +50,14 @@ namespace {
 
 // Rows per workgroup.  Large tiles hold more blocks in their tile (stored
 // once) and gather smaller halos, small ones give matrices of few rows enough
-// workgroups: back to back, FP64 / FP32 values, us per product of a
-// 27-neighbour grid with contacts at 4k, 32k, 64k, 110k and 262k rows
+// workgroups: back to back, FP64 / FP32 values, us per product in the halo
+// form of a 27-neighbour grid with contacts at 4k, 32k, 64k, 110k and 262k rows
 //   512 rows   13.5 / 10.8   16.0 / 11.5   17.2 / 12.3   19.4 / 13.9   43.8 / 24.8
 //   128 rows    8.1 /  7.3    9.7 /  8.1   13.7 / 10.0   22.7 / 18.2   49.7 / 39.2
 //    64 rows    7.1 /  6.5    9.8 /  7.6   18.4 / 14.7   27.1 / 25.5   62.2 / 56.0
+// The gather form keeps the same tiles: on the matrices that fall to it there,
+// with about 100 random blocks a row, 30k and 60k rows take 65 / 43 and 124 /
+// 75 us in 128-row tiles against 207 / 158 and 224 / 169 in 512-row ones.
 constexpr int kTileLarge = 512, kTileMid = 128, kTileSmall = 64;
 // up to 512 rows one tile holds the whole matrix (no halo); below these counts
 // the smaller tiles.  With FP32 values two workgroups share a CU, so past 512

@@ -45,6 +45,7 @@ ROWS = {
     "share_below": ([20000] + [25] * 800, 100),
     "share_above": ([20001] + [25] * 800, 100),
     "many_long": ([2100] * 40 + [64] * 12000, 3000),
+    "long_wide_blocks": ([5000, 4100, 3] + [60] * 400 + [2600], 20),
     "many_short": (list(np.random.default_rng(1).integers(0, 90, 3000)), 12),
 }
 
