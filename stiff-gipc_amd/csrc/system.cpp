@@ -776,7 +776,9 @@ int system_solve(sgipc_system* sys, const double* b, double* x, double* grad, co
             }
         });
         try {
-            // a pair puts about 7 triplets into the first row of its body
+            // a pair puts about 7 triplets into the first row of its body (16^3
+            // grid with 2 bodies: 300 pairs 0.21 ms by rows, 0.25 otherwise; 3k
+            // pairs 0.70 and 0.34)
             const bool long_rows = nb > 0 && 7L * d.n_pairs > 2048L * nb;
             sys->nnz = sys->conv.convert(s, sys->tvals.get(), sys->trows.get(), sys->tcols.get(), off, sys->n_sys,
                                          sys->bvals.get(), sys->brows.get(), sys->bcols.get(), sys->capacity, long_rows);
